@@ -259,7 +259,7 @@ int fused_ptr(L *h, const void *Uin, void *Uout, void *P, su2k::FusedCoef c, int
 // the half-field layout; links already in it are read in it.
 int flush_gen(L *h);
 int fused(L *h, int uin, int uout, void *P, su2k::FusedCoef c, int accum_row,
-          bool allow_half = false) {
+          bool allow_half = false, int *nparts = nullptr) {
   // pending device momenta: drawn inside a first P-then-U step with partial
   // sums, else by their own launch now
   const bool gen = h->gen_pending && P == h->P && uout >= 0 && accum_row >= 0;
@@ -276,6 +276,8 @@ int fused(L *h, int uin, int uout, void *P, su2k::FusedCoef c, int accum_row,
     fl.c.flags |= su2k::F_ACCUM;
     fl.partials = row(h, accum_row);
   }
+  if (nparts) *nparts = su2k::fused_blocks(h->geo);
+  fl.nparts = nparts;
   fl.in_half = h->half[uin];
   if (allow_half && su2k::fused_half_ok(h->group, h->prec, h->geo, fl.c.flags))
     fl.out_half = uout >= 0 ? 1 : 0;
@@ -473,6 +475,7 @@ struct IntegrateOut {
   bool first_accum = false;  // rows 0..2 hold kin_old/act/kin_new of the first step
   bool last_p_only = false;  // rows 3..5 hold the last momentum-only step sums
   int final_buf = -1;
+  int nb_first = 0, nb_last = 0;  // block partials per row of those sums
 };
 
 int run_integrator(L *h, int kind, size_t nsteps, double tau, size_t exponent,
@@ -510,12 +513,13 @@ int run_integrator(L *h, int kind, size_t nsteps, double tau, size_t exponent,
         CK(free_buf(h, {cur, protect.size() > 0 ? *protect.begin() : cur,
                         protect.size() > 1 ? *(protect.begin() + 1) : cur},
                     &out));
-        CK(fused(h, cur, out, h->P, c, acc_row, true));
+        CK(fused(h, cur, out, h->P, c, acc_row, true, acc_row >= 0 ? &io->nb_first : nullptr));
         cur = out;
         i += 2;
       } else {
         const int r = (accum && first) ? row_base + 0 : (accum && last_p) ? row_base + 3 : -1;
-        CK(fused(h, cur, -1, h->P, c, r, true));
+        int *nb = r < 0 ? nullptr : first ? &io->nb_first : &io->nb_last;
+        CK(fused(h, cur, -1, h->P, c, r, true, nb));
         if (accum && last_p && !first) io->last_p_only = true;
         i += 1;
       }
@@ -757,8 +761,8 @@ int su2gpu_create(su2gpu_lattice **out, int group, size_t Lx, size_t Ly, size_t 
   su2dev::geo_set_div(h->geo);
   hipError_t e = hipGetDevice(&h->device);
   if (e == hipSuccess) e = hipStreamCreateWithFlags(&h->stream, hipStreamNonBlocking);
-  const int nbf = su2k::fused_blocks(h->geo), nbs = su2k::sumsq_blocks((long)h->nlinks * h->nm);
-  h->row_stride = nbf > nbs ? nbf : nbs;
+  h->row_stride = std::max({su2k::fused_blocks(h->geo), su2k::plq_partials(group, precision, h->geo),
+                            su2k::sumsq_blocks((long)h->nlinks * h->nm)});
   if (e == hipSuccess) e = hipMalloc(&h->U[0], h->U_bytes);
   if (e == hipSuccess) e = hipMalloc(&h->U[1], h->U_bytes);
   if (e == hipSuccess) e = hipMalloc(&h->U[2], h->U_bytes);
@@ -1094,7 +1098,6 @@ static int trajectory_sums(L *h, int kind, size_t nsteps, double tau, size_t exp
                            std::initializer_list<int> protect, int rbase, int u_start,
                            long double *K_old, long double *S_old, long double *K_new,
                            long double *S_new, int *final_buf) {
-  const int nbf = su2k::fused_blocks(h->geo);
   const double w_t = h->aniso ? 1.0 / h->xi : 1.0, w_s = h->aniso ? h->xi : 1.0;
   const int pflags = h->aniso ? su2k::F_ANISO : 0;
   h->cur = u_start;
@@ -1130,9 +1133,9 @@ static int trajectory_sums(L *h, int kind, size_t nsteps, double tau, size_t exp
     CK(plaq_launch(h, cur, -1, w_t, w_s, 0, pflags, rbase + 7, &rl));
   }
   if (!io.last_p_only) CK(sumsq_launch(h, h->P, rbase + 8, &rl));
-  if (io.first_accum) CK(reduce_row(h, rbase + 0, nbf, &rl));
-  if (io.first_accum && h->prec == 0) CK(reduce_row(h, rbase + 1, nbf, &rl));
-  if (io.last_p_only) CK(reduce_row(h, rbase + 5, nbf, &rl));
+  if (io.first_accum) CK(reduce_row(h, rbase + 0, io.nb_first, &rl));
+  if (io.first_accum && h->prec == 0) CK(reduce_row(h, rbase + 1, io.nb_first, &rl));
+  if (io.last_p_only) CK(reduce_row(h, rbase + 5, io.nb_last, &rl));
   CK(reduce_rows(h, rl));
   CK(fetch_sums(h));
   *K_old = 0.5L * sum_of(h, rbase + 0);

@@ -666,7 +666,9 @@ static bool fast_geo_for(const Geo &g, FastGeo &f, bool wmu = false) {
 bool fused_half_ok(int group, int prec, const Geo &g, int flags) {
   if (group != 1 || prec != 0 || g.nd != 4) return false;
   if (fast_level() < 2 || fast_shape() == 1 || half_pref() == 0) return false;
-  if (flags & (F_PZERO | F_ROUND | F_ANISO | F_R32L | F_R32P)) return false;
+  if (flags & (F_PZERO | F_ROUND | F_R32L | F_R32P)) return false;
+  // the staple steps weight no planes in this layout
+  if ((flags & F_ANISO) && !plq_ok(group, prec, g, flags)) return false;
   if (fused_mode(g) == 0) return false;
   FastGeo f;
   return fast_geo_for(g, f);
@@ -1071,6 +1073,7 @@ static bool launch_first_step_gen(int group, int prec, const FusedLaunch &L, hip
 }
 
 bool launch_fused(int group, int prec, const FusedLaunch &L, hipStream_t st) {
+  if (fast_level() >= (prec == 0 ? 2 : 1) && launch_plq(group, prec, L, st)) return true;
   if (L.gen) {
     if (launch_first_step_gen(group, prec, L, st)) return true;
     launch_momenta_philox(prec, L.P, L.geo.V, L.geo.nd, group == 1 ? 3 : 1, L.c.gseed, L.c.gtraj,

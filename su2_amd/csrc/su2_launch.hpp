@@ -55,10 +55,19 @@ struct FusedLaunch {
   // c.gtraj (launch_momenta_philox), drawn inside the step where it walks t,
   // else by launch_momenta_philox before it
   int gen = 0;
+  // F_ACCUM: where the step keeps another number of block partials per row than
+  // fused_blocks(geo), it is written here
+  int *nparts = nullptr;
 };
 
 // false if a half-field layout was asked for where the step does not support it
 bool launch_fused(int group, int prec, const FusedLaunch &L, hipStream_t st);
+// the shared-plaquette step (su2_md_plq.hpp); false where it does not apply
+// (nothing launched).  plq_partials: its block partials per row, 0 likewise;
+// plq_ok: whether it applies with these flags
+bool launch_plq(int group, int prec, const FusedLaunch &L, hipStream_t st);
+int plq_partials(int group, int prec, const Geo &geo);
+bool plq_ok(int group, int prec, const Geo &geo, int flags);
 // whether a fused launch of this lattice with these flags runs the specialised
 // step that reads and writes the half-field layout (FP64 SU(2) d = 4,
 // isotropic, specialised launch layout)

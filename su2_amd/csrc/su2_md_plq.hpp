@@ -1,0 +1,658 @@
+// su2_md_plq.hpp -- the fused force / momentum / link update from shared
+// plaquettes (get_staples.hh:26-80, flat-gaugemonomial.hh:105-131,
+// update_momenta.hh:27-30, update_gauge.hh:11-14), SU(2) and U(1), d = 3, 4.
+//
+// The force of a link is a sum over its plaquettes, and a plaquette
+// P = a b c^+ d^+ (a = U_mu(x), b = U_nu(x+mu), c = U_mu(x+nu), d = U_nu(x))
+// serves four links:
+//   Im(U K):  a: +Im(P)            b: Im(b c^+ d^+ a)
+//             d: -Im(P)            c: Im(c b^+ a^+ d)
+// With M = a b and N = d c: P = M N^+, b c^+ d^+ a = b (N^+ a) and
+// c b^+ a^+ d = c (M^+ d).  A thread takes the site x, evaluates its planes
+// once and hands the b and c terms on to the sites x+mu and x+nu, where the
+// staple form evaluates every plaquette four times and loads 18 neighbour
+// links per link (10.75 with the links carried along t).  Here:
+//   * t: a thread walks the slices of a t-chunk upwards; the b terms of its
+//     planes (t, i) belong to its own next links and stay in registers, as do
+//     the links U_i(x+t) and U_1(x-1+t);
+//   * the two fastest directions: a block holds whole rows of the fastest one
+//     at one x (d = 4), links and terms are exchanged through LDS; a row whose
+//     neighbour row is in another block loads that row's links, and evaluates
+//     the terms it would have been handed itself;
+//   * x (d = 4): never in the block; the terms from x-1 are always evaluated
+//     here (three half planes, a quarter of the arithmetic).
+// d = 4: 13 link loads per site (3.25 per link) plus the edge rows'.
+//
+// Two barriers per slice; they wait for LDS only (asm, lgkmcnt), so global
+// loads stay in flight across them.
+//
+// What bounds it, and what it measured (steps with HIP events, against the
+// t-walk of the staple form, same box).  The staple form is bound by its link
+// requests (31 vector memory instructions per 64 links); this one has 15 and is
+// bound by the bytes beyond the L2 and the latency of two round trips per slice
+// (links; momenta and edge-row links, which are loaded together while the last
+// planes are evaluated).  FP64: 32^4 143 -> 107 us (565 MB beyond the L2, 5.3
+// TB/s), 48^4 784 -> 518 us (112 B per link at 4.6 TB/s), 40^4 386 -> 287 us,
+// 24^4 48.6 -> 38.9 us, momentum-only 32^4 115 -> 82 us.  FP32: 48^4 384 -> 285
+// us, 40^4 190 -> 151 us, 32^4 58.7 -> 55.7 us (VALU 60 % busy).  Loading the
+// next slice's first links during the update spills (FP64) and makes the next
+// slice wait for the update's stores, which share the counter of the loads:
+// 137 us at 32^4.
+#pragma once
+#include <algorithm>
+#include <cmath>
+
+#include "su2_md_fast.hpp"
+
+namespace su2k {
+
+// ------------------------------------------------------------------ layout --
+constexpr int PLQ_NT = 256;            // most threads of a block
+constexpr int PLQ_HALO = 64;           // longest row
+
+struct PlqGeo {
+  int L[4];      // extents t, x, y, z (1 above nd)
+  int str[4];    // site strides
+  int V, nd;
+  int vol3;      // sites of a t slice
+  int rpb;       // rows (of the fastest direction) per block
+  int nrows;     // rows per x plane (d = 4) or per slice (d = 3)
+  int nyb;       // blocks per x plane: ceil(nrows / rpb)
+  int nb3;       // blocks per slice
+  int Tc, nchunk;
+  uint32_t mLf;  // multiply-high divisors (fast_div): fastest extent, nyb, nb3
+  uint32_t mnyb, mnb3;
+};
+
+// block b of nblk, thread tid -> site of the slice, chunk, row and neighbours
+struct PlqSite {
+  bool active;
+  int o3;              // site within the slice
+  int t0, t1;          // slices [t0, t1)
+  int ux, dx;          // +-x neighbour offsets (d = 4)
+  int ur, dr;          // +- row direction
+  int uz, dz;          // +- fastest direction
+  bool rin;            // the row above is in this block
+  int lur, ldr;        // the row neighbours' thread; the halo's slot, -1 where in another block
+  int luz, ldz;        // the fastest direction's neighbours' thread
+};
+__host__ __device__ __forceinline__ PlqSite plq_site(const PlqGeo &g, uint32_t b, uint32_t nblk,
+                                                     uint32_t tid, uint32_t nt) {
+  PlqSite f;
+  // each XCD walks one contiguous eighth of the (chunk, block) sequence
+  const uint32_t xcd = b & 7u, local = b >> 3, per = nblk >> 3, rem = nblk & 7u;
+  const uint32_t lb = xcd * per + (xcd < rem ? xcd : rem) + local;
+  const uint32_t chunk = fast_div(lb, g.mnb3);
+  const uint32_t b3 = lb - chunk * (uint32_t)g.nb3;
+  f.t0 = (int)chunk * g.Tc;
+  f.t1 = f.t0 + g.Tc < g.L[0] ? f.t0 + g.Tc : g.L[0];
+  const uint32_t x = fast_div(b3, g.mnyb);
+  const int r0 = (int)(b3 - x * (uint32_t)g.nyb) * g.rpb;
+  const int Lf = g.L[g.nd - 1], Lr = g.nrows;
+  const int nr = Lr - r0 < g.rpb ? Lr - r0 : g.rpb;  // rows of this block
+  const uint32_t row = fast_div(tid, g.mLf);
+  const int z = (int)(tid - row * (uint32_t)Lf);
+  f.active = (int)row < nr;
+  const int r = f.active ? (int)row : 0;
+  const int y = r0 + r;
+  f.o3 = (int)x * (Lr * Lf) + y * Lf + z;
+  const int plane = Lr * Lf;
+  f.ux = ((int)x == g.L[1] - 1) ? -(g.L[1] - 1) * plane : plane;
+  f.dx = (x == 0) ? (g.L[1] - 1) * plane : -plane;
+  const int yu = (y == Lr - 1) ? 0 : y + 1, yd = (y == 0) ? Lr - 1 : y - 1;
+  f.ur = (yu - y) * Lf;
+  f.dr = (yd - y) * Lf;
+  f.uz = (z == Lf - 1) ? -(Lf - 1) : 1;
+  f.dz = (z == 0) ? Lf - 1 : -1;
+  f.rin = yu >= r0 && yu < r0 + nr;
+  f.lur = f.rin ? (int)tid + f.ur : (int)nt + z;
+  f.ldr = (yd >= r0 && yd < r0 + nr) ? (int)tid + f.dr : -1;
+  f.luz = (int)tid + f.uz;
+  f.ldz = (int)tid + f.dz;
+  if (!f.active) {
+    // a lane past the block's rows: reads as its first row's lane z, exchanges
+    // with itself, writes nothing
+    f.rin = true;
+    f.lur = f.ldr = f.luz = f.ldz = (int)tid;
+  }
+  return f;
+}
+
+inline uint32_t plq_blocks(const PlqGeo &g) { return (uint32_t)g.nb3 * (uint32_t)g.nchunk; }
+inline uint32_t plq_threads(const PlqGeo &g) {
+  return (uint32_t)((g.rpb * g.L[g.nd - 1] + 63) / 64 * 64);
+}
+
+// The rows of a block for extents L (t, x, y, z; nd = 3, 4); false where the
+// step does not apply.  rpb: the rows that waste the fewest lanes of at most
+// 256 threads, fewer edge rows breaking ties.
+inline bool make_plq_rows(const int L[4], int nd, int V, PlqGeo &g) {
+  if (nd < 3 || nd > 4) return false;
+  for (int k = 0; k < 4; ++k) g.L[k] = L[k];
+  g.nd = nd;
+  g.V = V;
+  g.str[3] = 1;
+  g.str[2] = L[3];
+  g.str[1] = L[2] * L[3];
+  g.str[0] = L[1] * L[2] * L[3];
+  g.vol3 = g.str[0];
+  const int Lf = L[nd - 1];
+  g.nrows = L[nd - 2];
+  if (Lf > PLQ_HALO || Lf < 2) return false;
+  const uint64_t two32 = 1ull << 32;
+  if ((uint64_t)V * 32u >= two32) return false;  // 32-bit byte offsets in a plane
+  double best = 0.0;
+  g.rpb = 0;
+  for (int r = 1; r <= g.nrows && r * Lf <= PLQ_NT; ++r) {
+    const int nyb = (g.nrows + r - 1) / r, nt = (r * Lf + 63) / 64 * 64;
+    // useful rows per lane, less the edge rows' terms (a fifth of a row each,
+    // none where the block holds every row)
+    const double eff = (double)g.nrows * Lf / ((double)nyb * nt) /
+                       (1.0 + (nyb > 1 ? 0.2 / r : 0.0));
+    if (eff > best * 1.0001) {
+      best = eff;
+      g.rpb = r;
+    }
+  }
+  if (g.rpb < 1) return false;
+  g.nyb = (g.nrows + g.rpb - 1) / g.rpb;
+  g.nb3 = g.nyb * (nd == 4 ? L[1] : 1);
+  g.mLf = fast_div_magic((uint32_t)Lf);
+  return true;
+}
+
+// The t-chunks where `percu` blocks are resident on each of `cus` CUs.  A slice
+// of a resident round costs a latency and a share per resident wave, in the
+// ratio 2 : 1 (FP32 32^4, measured: chunks of 8 slices, 8 waves per CU, 55.7 us;
+// of 6, 12 waves, 59.6; of 4, two rounds, 61.9; FP64 24^4: 4 slices 39, 3 slices
+// 43.7, 2 slices 43.2 us), a chunk's first slice a third more (the terms of
+// the slice below it).
+inline bool make_plq_chunks(int percu, int cus, PlqGeo &g) {
+  const int waves = (g.rpb * g.L[g.nd - 1] + 63) / 64;
+  double cost = 1e300;
+  g.Tc = 1;
+  for (int Tc = 1; Tc <= g.L[0]; ++Tc) {
+    const int nc = (g.L[0] + Tc - 1) / Tc;
+    double c = 0.0;
+    for (long left = (long)g.nb3 * nc; left > 0; left -= (long)percu * cus) {
+      const long b = std::min<long>((left + cus - 1) / cus, percu);
+      c += (Tc + 0.35) * (2.0 + (double)(b * waves));
+      if (c > cost) break;
+    }
+    if (c < cost * 0.999) {
+      cost = c;
+      g.Tc = Tc;
+    }
+  }
+  g.nchunk = (g.L[0] + g.Tc - 1) / g.Tc;
+  if ((uint64_t)g.nb3 * g.nchunk * g.nb3 >= (1ull << 32)) return false;
+  g.mnyb = fast_div_magic((uint32_t)g.nyb);
+  g.mnb3 = fast_div_magic((uint32_t)g.nb3);
+  return true;
+}
+
+// ------------------------------------------------------------ the algebra --
+template <typename T> struct pv3 {
+  T k[3];
+};
+
+// Im(u v) in momentum order (bi, br, ai)
+template <typename T> __device__ __forceinline__ pv3<T> qim(const quat<T> &u, const quat<T> &v) {
+  pv3<T> r;
+  r.k[2] = fma(u.ar, v.ai, fma(u.ai, v.ar, fma(-u.bi, v.br, u.br * v.bi)));
+  r.k[1] = fma(u.ar, v.br, fma(-u.ai, v.bi, fma(u.br, v.ar, u.bi * v.ai)));
+  r.k[0] = fma(u.ar, v.bi, fma(u.ai, v.br, fma(u.bi, v.ar, -(u.br * v.ai))));
+  return r;
+}
+template <typename T> __device__ __forceinline__ double qre(const quat<T> &u, const quat<T> &v) {
+  return double(fma(u.ar, v.ar, -fma(u.ai, v.ai, fma(u.br, v.br, u.bi * v.bi))));
+}
+
+// SU(2): terms are three reals
+template <typename T_> struct PlqSU2 {
+  using T = T_;
+  using link = quat<T>;
+  static constexpr int NM = 3;
+  using V = pv3<T>;
+  // B, C: whether the b / c term is wanted; RE: re += w ReTr(P) / 2
+  template <bool B, bool C, bool RE>
+  __device__ static void plane(const link &a, const link &b, const link &c, const link &d, V &v0,
+                               V &vb, V &vc, double w, double &re) {
+    const link M = qmul_fma(a, b), N = qmul_fma(d, c);
+    v0 = qim(M, qdag(N));
+    if (RE) re = fma(w, qre(M, qdag(N)), re);
+    if (B) vb = qim(b, qmul_fma(qdag(N), a));
+    if (C) vc = qim(c, qmul_fma(qdag(M), d));
+  }
+  __device__ static V lowb(const link &a, const link &b, const link &c, const link &d) {
+    return qim(b, qmul_fma(qdag(qmul_fma(d, c)), a));
+  }
+  __device__ static V lowc(const link &a, const link &b, const link &c, const link &d) {
+    return qim(c, qmul_fma(qdag(qmul_fma(a, b)), d));
+  }
+};
+
+// ------------------------------------------------------------------- memory --
+__device__ __forceinline__ void plq_barrier() {
+  // LDS writes done, then the barrier; global loads may stay in flight
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+
+// The exchange in LDS: one record per thread (and of a halo row) with the nd
+// links, one per thread with the 2 (nd - 1) terms.  The offsets within a record
+// are immediates of the LDS instructions, so a thread needs one address per
+// neighbour; records are odd multiples of 16 B (links) or 8 B apart modulo the
+// banks, so the lanes of an access spread over them.
+template <class G, int ND> constexpr int plq_lrec() {
+  return (ND * (int)sizeof(typename G::link) / 16 | 1) * 16;
+}
+template <class G, int ND> constexpr int plq_vrec() {
+  return (2 * (ND - 1) * G::NM | 1) * (int)sizeof(typename G::T);
+}
+__device__ __forceinline__ void plq_put(char *rec, int k, const quat<double> &q) {
+  su2_d2 *p = (su2_d2 *)rec + 2 * k;
+  p[0] = su2_d2{q.ar, q.ai};
+  p[1] = su2_d2{q.br, q.bi};
+}
+__device__ __forceinline__ void plq_get(const char *rec, int k, quat<double> &q) {
+  const su2_d2 *p = (const su2_d2 *)rec + 2 * k;
+  const su2_d2 a = p[0], b = p[1];
+  q = quat<double>{a.x, a.y, b.x, b.y};
+}
+__device__ __forceinline__ void plq_put(char *rec, int k, const quat<float> &q) {
+  ((su2_f4 *)rec)[k] = su2_f4{q.ar, q.ai, q.br, q.bi};
+}
+__device__ __forceinline__ void plq_get(const char *rec, int k, quat<float> &q) {
+  const su2_f4 a = ((const su2_f4 *)rec)[k];
+  q = quat<float>{a.x, a.y, a.z, a.w};
+}
+template <typename T> __device__ __forceinline__ void plq_putv(char *rec, int k, const pv3<T> &v) {
+  T *p = (T *)rec + 3 * k;
+  p[0] = v.k[0];
+  p[1] = v.k[1];
+  p[2] = v.k[2];
+}
+template <typename T>
+__device__ __forceinline__ void plq_getv(const char *rec, int k, pv3<T> &v) {
+  const T *p = (const T *)rec + 3 * k;
+  v.k[0] = p[0];
+  v.k[1] = p[1];
+  v.k[2] = p[2];
+}
+template <class G, int ND> size_t plq_lds(const PlqGeo &g) {
+  const size_t nt = plq_threads(g);
+  return (nt + g.L[g.nd - 1]) * plq_lrec<G, ND>() + nt * plq_vrec<G, ND>();
+}
+
+// the values are complete here: keeps the compiler from sinking their arithmetic
+// past later loads, which would hold its operands in registers
+template <typename T> __device__ __forceinline__ void plq_pin(T (&v)[3]) {
+  asm volatile("" : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]));
+}
+
+// acc += w v
+template <typename V> __device__ __forceinline__ void plq_add(double (&acc)[3], double w, const V &v) {
+#pragma unroll
+  for (int k = 0; k < 3; ++k) acc[k] = fma(w, double(v.k[k]), acc[k]);
+}
+
+// cos a and sin(a)/a of the FP64 update for x = a^2: Taylor series in y to y^8
+// (remainders y^9 / 18! <= 1.6e-16 and y^9 / 19! for y <= 1, at most an ulp
+// with the Horner roundings), y = x where x <= 1; beyond that y = r^2 with
+// a = q pi/2 + r, |r| <= pi/4 (pi/2 in two parts, the first of 33 bits, so that
+// q times it is exact for the q < 2^17 that occur).
+__device__ __forceinline__ void cos_sinc_fp64(double x, double &c, double &s) {
+  double y = x, r = 0.0, q = 0.0;
+  const bool big = !(x <= 1.0);
+  if (big) {
+    double al = sqrt(x);
+    if (al > 1e5) al = fmod(al, 6.283185307179586477);
+    q = rint(al * 0.6366197723675813431);
+    r = fma(-q, 6.07710050650619224932e-11, fma(-q, 1.57079632673412561417, al));
+    y = r * r;
+  }
+  double t = fma(y, 1.0 / 20922789888000.0, -1.0 / 87178291200.0);
+  double u = fma(y, 1.0 / 355687428096000.0, -1.0 / 1307674368000.0);
+  t = fma(y, t, 1.0 / 479001600);
+  u = fma(y, u, 1.0 / 6227020800.0);
+  t = fma(y, t, -1.0 / 3628800);
+  u = fma(y, u, -1.0 / 39916800);
+  t = fma(y, t, 1.0 / 40320);
+  u = fma(y, u, 1.0 / 362880);
+  t = fma(y, t, -1.0 / 720);
+  u = fma(y, u, -1.0 / 5040);
+  t = fma(y, t, 1.0 / 24);
+  u = fma(y, u, 1.0 / 120);
+  t = fma(y, t, -0.5);
+  u = fma(y, u, -1.0 / 6);
+  c = fma(y, t, 1.0);
+  s = fma(y, u, 1.0);
+  if (big) {
+    const int j = (int)q;
+    const double sr = r * s;
+    const double sn = (j & 1) ? c : sr, cs = (j & 1) ? sr : c;
+    c = ((j + 1) & 2) ? -cs : cs;
+    s = ((j & 2) ? -sn : sn) / sqrt(x);
+  }
+}
+
+// element i + k V of a plane triple as one scalar base + 32-bit byte offset
+// (3 V sizeof(T) < 2^32): the three planes share the base's registers
+template <typename T> __device__ __forceinline__ uint32_t plq_off(uint32_t V, int k, uint32_t i) {
+  return (i + (uint32_t)k * V) * (uint32_t)sizeof(T);
+}
+
+// momentum and link update of one link from G = Im(U K):
+// P' = P - 2 coef ep G rounded once, U' = exp(eu P') U
+template <typename T, bool W, int NT, class UO>
+__device__ __forceinline__ void plq_update(const quat<T> &u, const double (&G)[3],
+                                           const T (&pi)[3], T (&pn)[3], T *Pw, uint32_t V, UO Uo,
+                                           uint32_t s, const FusedCoef &c) {
+  const double f = 2.0 * c.coef * c.ep;
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    pn[k] = T(fma(-f, G[k], double(pi[k])));
+    T *q = (T *)((char *)Pw + plq_off<T>(V, k, s));
+    if (NT) __builtin_nontemporal_store(pn[k], q);
+    else *q = pn[k];
+  }
+  if constexpr (W) {
+    const double e0 = c.eu * double(pn[0]), e1 = c.eu * double(pn[1]), e2 = c.eu * double(pn[2]);
+    const double x = fma(e0, e0, fma(e1, e1, e2 * e2));
+    double cs, sn;
+    if constexpr (sizeof(T) == 4) cos_sinc_step(x, cs, sn);
+    else cos_sinc_fp64(x, cs, sn);
+    quat<double> n = qmul_fma(quat<double>{cs, sn * e2, sn * e1, sn * e0}, to_d(u));
+    if constexpr (sizeof(T) == 4) {
+      if (c.flags & F_RESTORE) {
+        // 1/sqrt(1 + d) as in md_su2_update
+        const double d = fma(n.ar, n.ar, fma(n.ai, n.ai, fma(n.br, n.br, fma(n.bi, n.bi, -1.0))));
+        const double r = (fabs(d) < 1e-4) ? 1.0 + d * (-0.5 + 0.375 * d) : 1.0 / sqrt(1.0 + d);
+        n = qscale(r, n);
+      }
+    }
+    stq<NT>(Uo, s, quat<T>{T(n.ar), T(n.ai), T(n.br), T(n.bi)});
+  }
+}
+
+// ------------------------------------------------------------------ the step --
+// W: write the new links (false: momenta alone); ACC: block partials of
+// |P_in|^2, ReTr(U K) and |P_out|^2.  pin / pout may be the same field.
+// flags: F_PZERO (momenta read as zero), F_RESTORE; w_t / w_s weight the planes
+// (1 where isotropic: fma with 1 is the plain sum).  GEN: the momenta are drawn
+// (Philox counter of k_momenta_philox) instead of loaded.  NT: 0 ordinary
+// accesses, 2 non-temporal stores and momentum loads.
+template <class G, int ND, bool W, bool ACC, bool GEN, int NT, class UI, class UO>
+__global__ __launch_bounds__(PLQ_NT, sizeof(typename G::T) == 8 ? 2 : 3) void k_md_plq(
+    UI Uin, UO Uout, const typename G::T *Pin, typename G::T *Pout, PlqGeo g, FusedCoef c,
+    double *__restrict__ partials, int pstride) {
+  using T = typename G::T;
+  using link = typename G::link;
+  using Vc = typename G::V;
+  extern __shared__ __align__(16) char smem[];
+  const int nt = (int)blockDim.x, tid = (int)threadIdx.x;
+  constexpr int R = ND - 2, Z = ND - 1;              // row and fastest direction
+  constexpr bool X4 = ND == 4;
+  const PlqSite f = plq_site(g, blockIdx.x, gridDim.x, (uint32_t)tid, (uint32_t)nt);
+  const size_t V = (size_t)g.V;
+  // LDS records: own, of the row above (or the halo's), of x+z; the terms' of
+  // own, of the row below, of x-z
+  constexpr int LREC = plq_lrec<G, ND>(), VREC = plq_vrec<G, ND>();
+  char *const lv0 = smem + (nt + g.L[Z]) * LREC;
+  char *const lown = smem + tid * LREC, *const lrow = smem + f.lur * LREC,
+             *const lz = smem + f.luz * LREC;
+  char *const vown = lv0 + tid * VREC, *const vrow = lv0 + f.ldr * VREC,
+             *const vz = lv0 + f.ldz * VREC;
+  UI U[ND];
+#pragma unroll
+  for (int m = 0; m < ND; ++m) U[m] = fld_add(Uin, (size_t)m * V);
+  const bool rin = f.rin, din = f.ldr >= 0;
+  const bool edge = __builtin_amdgcn_readfirstlane((int)(__ballot(!din) != 0)) != 0;
+  const double wt = c.w_t, ws = c.w_s;
+  double sums[3] = {0.0, 0.0, 0.0};
+  double re = 0.0;
+
+  link own[ND], xl;
+  Vc carry[ND];  // [1 ..]: the b terms of the planes (t, i) of the slice below
+  int s = f.t0 * g.vol3 + f.o3;
+  auto up_t = [&](int t) { return t == g.L[0] - 1 ? -(g.L[0] - 1) * g.vol3 : g.vol3; };
+  {
+    const int dt = f.t0 == 0 ? (g.L[0] - 1) * g.vol3 : -g.vol3;
+    const link a = ldq(U[0], (uint32_t)(s + dt));
+    const int up[4] = {0, X4 ? f.ux : f.ur, X4 ? f.ur : f.uz, f.uz};
+    if (X4) xl = ldq(U[1], (uint32_t)(s + f.dx));
+#pragma unroll
+    for (int i = 1; i < ND; ++i) {
+      own[i] = ldq(U[i], (uint32_t)s);
+      const link cc = ldq(U[0], (uint32_t)(s + dt + up[i]));
+      const link dd = ldq(U[i], (uint32_t)(s + dt));
+      carry[i] = G::lowb(a, own[i], cc, dd);
+    }
+  }
+  for (int t = f.t0; t < f.t1; ++t) {
+    const int ut = up_t(t);
+    double acc[ND][3];
+    link nx[ND], ux[ND], xlt;
+    {
+      // every load of the slice but the momenta's, in the order of use
+      link lx[ND], lxu[ND];
+      own[0] = ldq(U[0], (uint32_t)s);
+      if constexpr (X4) {
+        lx[0] = ldq(U[0], (uint32_t)(s + f.dx));
+        xlt = ldq(U[1], (uint32_t)(s + f.dx + ut));
+        lx[2] = ldq(U[2], (uint32_t)(s + f.dx));
+        lxu[2] = ldq(U[1], (uint32_t)(s + f.dx + f.ur));
+        lx[3] = ldq(U[3], (uint32_t)(s + f.dx));
+        lxu[3] = ldq(U[1], (uint32_t)(s + f.dx + f.uz));
+      }
+      if (!rin) {
+        // the links of the row above, where it is in another block, for the halo
+        link h[ND];
+#pragma unroll
+        for (int m = 0; m < ND; ++m)
+          if (m != R) h[m] = ldq(U[m], (uint32_t)(s + f.ur));
+#pragma unroll
+        for (int m = 0; m < ND; ++m)
+          if (m != R) plq_put(lrow, m, h[m]);
+      }
+#pragma unroll
+      for (int i = 1; i < ND; ++i) nx[i] = ldq(U[i], (uint32_t)(s + ut));
+      if constexpr (X4) {
+        ux[2] = ldq(U[2], (uint32_t)(s + f.ux));
+        ux[3] = ldq(U[3], (uint32_t)(s + f.ux));
+        ux[0] = ldq(U[0], (uint32_t)(s + f.ux));
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int m = 0; m < ND; ++m) plq_put(lown, m, own[m]);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int i = 1; i < ND; ++i)
+#pragma unroll
+        for (int k = 0; k < 3; ++k) acc[i][k] = wt * double(carry[i].k[k]);
+      acc[0][0] = acc[0][1] = acc[0][2] = 0.0;
+      if constexpr (X4) {
+        plq_add(acc[0], wt, G::lowc(lx[0], xlt, own[0], xl));        // (t, x) at x-1
+        plq_add(acc[2], ws, G::lowb(xl, own[2], lxu[2], lx[2]));     // (x, y)
+        plq_add(acc[3], ws, G::lowb(xl, own[3], lxu[3], lx[3]));     // (x, z)
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int m = 0; m < ND; ++m) plq_pin(acc[m]);
+    }
+    plq_barrier();
+    T pi[ND][3];
+    link eR, e0, eRt, eZ, eRz, eX, eRx;
+    {
+      Vc v0, vb, vc;
+      double ret = 0.0, res = 0.0;
+      link p, q;
+      // (r, z): b term to U_z(x+r), c term to U_r(x+z)
+      plq_get(lrow, Z, p);
+      plq_get(lz, R, q);
+      G::template plane<true, true, ACC>(own[R], p, q, own[Z], v0, vb, vc, 1.0, res);
+      plq_add(acc[R], ws, v0);
+      plq_add(acc[Z], -ws, v0);
+      plq_putv(vown, ND - 2, vb);
+      plq_putv(vown, 2 * (ND - 1) - 1, vc);
+      __builtin_amdgcn_sched_barrier(0);
+      // (t, r): c term to U_t(x+r); (t, z): to U_t(x+z)
+      plq_get(lrow, 0, q);
+      G::template plane<true, true, ACC>(own[0], nx[R], q, own[R], v0, vb, vc, 1.0, ret);
+      plq_add(acc[0], wt, v0);
+      plq_add(acc[R], -wt, v0);
+      carry[R] = vb;
+      plq_putv(vown, 0, vc);
+      __builtin_amdgcn_sched_barrier(0);
+      plq_get(lz, 0, q);
+      G::template plane<true, true, ACC>(own[0], nx[Z], q, own[Z], v0, vb, vc, 1.0, ret);
+      plq_add(acc[0], wt, v0);
+      plq_add(acc[Z], -wt, v0);
+      carry[Z] = vb;
+      plq_putv(vown, ND - 1, vc);
+      __builtin_amdgcn_sched_barrier(0);
+      if constexpr (X4) {
+        plq_get(lrow, 1, q);
+        G::template plane<false, true, ACC>(own[1], ux[2], q, own[2], v0, vb, vc, 1.0, res);
+        plq_add(acc[1], ws, v0);
+        plq_add(acc[2], -ws, v0);
+        plq_putv(vown, 1, vc);
+        __builtin_amdgcn_sched_barrier(0);
+        plq_get(lz, 1, q);
+        G::template plane<false, true, ACC>(own[1], ux[3], q, own[3], v0, vb, vc, 1.0, res);
+        plq_add(acc[1], ws, v0);
+        plq_add(acc[3], -ws, v0);
+        plq_putv(vown, ND, vc);
+        __builtin_amdgcn_sched_barrier(0);
+        G::template plane<true, false, ACC>(own[0], nx[1], ux[0], own[1], v0, vb, vc, 1.0, ret);
+        plq_add(acc[0], wt, v0);
+        plq_add(acc[1], -wt, v0);
+        carry[1] = vb;
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      if (ACC) {
+        if (f.active) re += fma(wt, ret, ws * res);
+        asm volatile("" : "+v"(re));
+      }
+#pragma unroll
+      for (int m = 0; m < ND; ++m) plq_pin(acc[m]);
+#pragma unroll
+      for (int i = 1; i < ND; ++i) plq_pin(carry[i].k);
+      // the momenta, in flight across the barrier
+      if constexpr (GEN) {
+#pragma unroll
+        for (int m = 0; m < ND; ++m) {
+          T z[4];
+          philox_normals4<T>((uint32_t)(s * ND + m), (uint32_t)(c.gtraj & 0xffffffffu),
+                             (uint32_t)(c.gtraj >> 32), c.gseed, z);
+#pragma unroll
+          for (int k = 0; k < 3; ++k) pi[m][k] = z[k];
+        }
+      } else if (c.flags & F_PZERO) {
+#pragma unroll
+        for (int m = 0; m < ND; ++m)
+#pragma unroll
+          for (int k = 0; k < 3; ++k) pi[m][k] = T(0);
+      } else {
+#pragma unroll
+        for (int m = 0; m < ND; ++m) {
+          const char *p = (const char *)(Pin + (size_t)(m * 3) * V);
+#pragma unroll
+          for (int k = 0; k < 3; ++k) {
+            const T *q = (const T *)(p + plq_off<T>((uint32_t)g.V, k, (uint32_t)s));
+            if constexpr (NT == 2) pi[m][k] = __builtin_nontemporal_load(q);
+            else pi[m][k] = *q;
+          }
+        }
+      }
+      // links of the row below, where it is in another block (the waves that
+      // hold such a row)
+      if (edge) {
+        const int sr = s + f.dr;
+        eR = ldq(U[R], (uint32_t)sr);
+        e0 = ldq(U[0], (uint32_t)sr);
+        eRt = ldq(U[R], (uint32_t)(sr + ut));
+        eZ = ldq(U[Z], (uint32_t)sr);
+        eRz = ldq(U[R], (uint32_t)(sr + f.uz));
+        if constexpr (X4) {
+          eX = ldq(U[1], (uint32_t)sr);
+          eRx = ldq(U[R], (uint32_t)(sr + f.ux));
+        }
+      }
+    }
+    plq_barrier();
+    {
+      Vc v;
+      // from x-z: U_t, U_x (d = 4), U_r
+      plq_getv(vz, ND - 1, v);
+      plq_add(acc[0], wt, v);
+      if constexpr (X4) {
+        plq_getv(vz, ND, v);
+        plq_add(acc[1], ws, v);
+      }
+      plq_getv(vz, 2 * (ND - 1) - 1, v);
+      plq_add(acc[R], ws, v);
+      if (din) {
+        // from x-r: U_t, U_x (d = 4), U_z
+        plq_getv(vrow, 0, v);
+        plq_add(acc[0], wt, v);
+        if constexpr (X4) {
+          plq_getv(vrow, 1, v);
+          plq_add(acc[1], ws, v);
+        }
+        plq_getv(vrow, ND - 2, v);
+        plq_add(acc[Z], ws, v);
+      }
+      if (edge) {
+        // the terms they give, for the lanes whose row below they are
+        const double wte = din ? 0.0 : wt, wse = din ? 0.0 : ws;
+        plq_add(acc[0], wte, G::lowc(e0, eRt, own[0], eR));           // (t, r): c is U_t(x)
+        plq_add(acc[Z], wse, G::lowb(eR, own[Z], eRz, eZ));           // (r, z): b is U_z(x)
+        if constexpr (X4)
+          plq_add(acc[1], wse, G::lowc(eX, eRx, own[1], eR));         // (x, r): c is U_x(x)
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      if (f.active) {
+#pragma unroll
+        for (int m = 0; m < ND; ++m) {
+          T pn[3];
+          plq_update<T, W, NT>(own[m], acc[m], pi[m], pn,
+                               Pout + (size_t)(m * 3) * V, (uint32_t)g.V,
+                               fld_add(Uout, (size_t)m * V), (uint32_t)s, c);
+          if (ACC) {
+            sums[0] += sq3(pi[m][0], pi[m][1], pi[m][2]);
+            sums[2] += sq3(pn[0], pn[1], pn[2]);
+          }
+        }
+      }
+      if (ACC) plq_pin(sums);
+      // the next slice
+#pragma unroll
+      for (int i = 1; i < ND; ++i) own[i] = nx[i];
+      if (X4) xl = xlt;
+      s += ut;
+    }
+  }
+  if (ACC) {
+    // ReTr(U K) of every link: a plaquette's 2 Re(P) once for each of its four
+    sums[1] = 8.0 * re;
+    __syncthreads();
+    double *l3 = (double *)smem;
+    const int lane = tid & 63, wv = tid >> 6, nw = nt >> 6;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      double v = sums[k];
+#pragma unroll
+      for (int o = 32; o > 0; o >>= 1) v += __shfl_down(v, o, 64);
+      if (lane == 0) l3[k * 4 + wv] = v;
+    }
+    __syncthreads();
+    if (tid < 3) {
+      double v = 0.0;
+      for (int i = 0; i < nw; ++i) v += l3[tid * 4 + i];
+      partials[(size_t)tid * pstride + blockIdx.x] = v;
+    }
+  }
+}
+
+}  // namespace su2k

@@ -1,0 +1,107 @@
+// su2_plq.hip -- launches of the shared-plaquette step (su2_md_plq.hpp).
+#include "su2_md_plq.hpp"
+
+namespace su2k {
+
+namespace {
+
+constexpr int CUS = 256;  // MI355X
+
+// resident blocks on a CU: registers leave room for 8 waves (FP64, 2 per SIMD)
+// or 12 (FP32), LDS for 160 KB
+template <class G, int ND> int plq_percu(const PlqGeo &g) {
+  const int waves = (int)plq_threads(g) / 64, lds = (int)plq_lds<G, ND>(g);
+  return std::max(1, std::min((sizeof(typename G::T) == 8 ? 8 : 12) / waves, 160 * 1024 / lds));
+}
+
+// The layout, or false where the staple steps are taken instead.  Below 32768
+// (FP64) and 98304 sites (FP32) those are as fast or faster: a launch is bound by
+// its chain of memory round trips, of which this step has two more (FP64 step
+// with events, this / staples: 12^4 10.2 / 9.8, 16^4 12.3 / 13.1, d = 3 32^3 8.5 /
+// 8.7 us; FP32: 16^4 10.5 / 9.7, 20^4 15.8 / 16.2, d = 3 21 59 79 10.1 / 10.3 us).
+bool plq_geo_for(int group, int prec, const Geo &geo, PlqGeo &g) {
+  if (group != 1 || geo.V < (prec == 0 ? 32768 : 98304)) return false;
+  if (!make_plq_rows(geo.L, geo.nd, geo.V, g)) return false;
+  const int percu = prec == 0 ? (geo.nd == 4 ? plq_percu<PlqSU2<double>, 4>(g)
+                                             : plq_percu<PlqSU2<double>, 3>(g))
+                              : (geo.nd == 4 ? plq_percu<PlqSU2<float>, 4>(g)
+                                             : plq_percu<PlqSU2<float>, 3>(g));
+  return make_plq_chunks(percu, CUS, g);
+}
+
+template <class G, int ND, bool W, bool ACC, bool GEN, int NT, class UI, class UO>
+void go(UI ui, UO uo, const FusedLaunch &L, const PlqGeo &g, hipStream_t st) {
+  using T = typename G::T;
+  const unsigned lds = (unsigned)plq_lds<G, ND>(g);
+  hipLaunchKernelGGL((k_md_plq<G, ND, W, ACC, GEN, NT, UI, UO>), dim3(plq_blocks(g)),
+                     dim3(plq_threads(g)), lds, st, ui, uo, (const T *)L.P,
+                     (T *)(L.Pout ? L.Pout : L.P), g, L.c, L.partials, L.pstride);
+}
+
+template <class G, int ND, class UI, class UO>
+void go_wa(UI ui, UO uo, const FusedLaunch &L, const PlqGeo &g, bool nt, hipStream_t st) {
+  const bool acc = (L.c.flags & F_ACCUM) != 0;
+#define SU2_GO(W, A, GN)                                       \
+  do {                                                         \
+    if (nt) go<G, ND, W, A, GN, 2, UI, UO>(ui, uo, L, g, st);  \
+    else go<G, ND, W, A, GN, 0, UI, UO>(ui, uo, L, g, st);     \
+  } while (0)
+  if (L.Uout) {
+    if (acc && L.gen) SU2_GO(true, true, true);
+    else if (acc) SU2_GO(true, true, false);
+    else SU2_GO(true, false, false);
+  } else {
+    if (acc) SU2_GO(false, true, false);
+    else SU2_GO(false, false, false);
+  }
+#undef SU2_GO
+}
+
+}  // namespace
+
+bool plq_ok(int group, int prec, const Geo &geo, int flags) {
+  PlqGeo g;
+  return !(flags & (F_ROUND | F_R32L | F_R32P)) && plq_geo_for(group, prec, geo, g);
+}
+
+int plq_partials(int group, int prec, const Geo &geo) {
+  PlqGeo g;
+  return plq_geo_for(group, prec, geo, g) ? (int)plq_blocks(g) : 0;
+}
+
+bool launch_plq(int group, int prec, const FusedLaunch &L, hipStream_t st) {
+  if (L.c.flags & (F_ROUND | F_R32L | F_R32P)) return false;
+  if (L.gen && !(L.Uout && (L.c.flags & F_ACCUM))) return false;
+  if (L.in_half && L.Uout && !L.out_half) return false;  // half -> record steps are not built
+  PlqGeo g;
+  if (!plq_geo_for(group, prec, L.geo, g)) return false;
+  if (L.nparts) *L.nparts = (int)plq_blocks(g);
+  // Non-temporal stores and momentum loads where the two link fields and the
+  // momenta exceed the 256 MB Infinity Cache: FP64 32^4 (369 MB) 106.9 against
+  // 109.4 us with the stores alone and 124 with neither, FP32 48^4 284.9 /
+  // 293.5 / 315; below, FP64 24^4 (117 MB) 43.5 with them and 38.8 without
+  const double fields = (double)L.geo.nd * L.geo.V * (prec == 0 ? 88.0 : 44.0);
+  const bool nt = fields > 256.0 * 1024 * 1024;
+  if (prec == 0 && L.geo.nd == 4) {
+    const size_t nl = 4 * (size_t)L.geo.V;
+    const su2_d2 *ia = (const su2_d2 *)L.Uin;
+    su2_d2 *oa = (su2_d2 *)L.Uout;
+    const QHalf hin{ia, ia + nl};
+    const QHalfW hout{oa, oa ? oa + nl : nullptr};
+    const quat<double> *rin = (const quat<double> *)L.Uin;
+    if (L.in_half) go_wa<PlqSU2<double>, 4>(hin, hout, L, g, nt, st);
+    else if (L.out_half) go_wa<PlqSU2<double>, 4>(rin, hout, L, g, nt, st);
+    else go_wa<PlqSU2<double>, 4>(rin, (quat<double> *)L.Uout, L, g, nt, st);
+    return true;
+  }
+  if (L.in_half || L.out_half) return false;
+#define SU2_PLQ(T, ND) \
+  go_wa<PlqSU2<T>, ND>((const quat<T> *)L.Uin, (quat<T> *)L.Uout, L, g, nt, st)
+  if (prec == 0) SU2_PLQ(double, 3);
+  else if (L.geo.nd == 4) SU2_PLQ(float, 4);
+  else SU2_PLQ(float, 3);
+#undef SU2_PLQ
+  return true;
+}
+
+}  // namespace su2k
