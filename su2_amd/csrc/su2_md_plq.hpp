@@ -34,7 +34,10 @@
 // planes are evaluated).  FP64: 32^4 143 -> 107 us (565 MB beyond the L2, 5.3
 // TB/s), 48^4 784 -> 518 us (112 B per link at 4.6 TB/s), 40^4 386 -> 287 us,
 // 24^4 48.6 -> 38.9 us, momentum-only 32^4 115 -> 82 us.  FP32: 48^4 384 -> 285
-// us, 40^4 190 -> 151 us, 32^4 58.7 -> 55.7 us (VALU 60 % busy).  Loading the
+// us, 40^4 190 -> 151 us, 32^4 58.7 -> 55.7 us (VALU 60 % busy).  U(1), where the
+// staple form takes seven sine / cosine pairs per link and this one six sines per
+// site and three for x-1: FP64 24^4 33.8 -> 17.8 us, 32^4 85.5 -> 35.2 us, d = 3
+// 64^3 17.8 -> 10.9 us; FP32 32^4 46.7 -> 24.3 us.  Loading the
 // next slice's first links during the update spills (FP64) and makes the next
 // slice wait for the update's stores, which share the counter of the loads:
 // 137 us at 32^4.
@@ -48,7 +51,7 @@ namespace su2k {
 
 // ------------------------------------------------------------------ layout --
 constexpr int PLQ_NT = 256;            // most threads of a block
-constexpr int PLQ_HALO = 64;           // longest row
+constexpr int PLQ_ROW = 128;           // longest row
 
 struct PlqGeo {
   int L[4];      // extents t, x, y, z (1 above nd)
@@ -138,7 +141,7 @@ inline bool make_plq_rows(const int L[4], int nd, int V, PlqGeo &g) {
   g.vol3 = g.str[0];
   const int Lf = L[nd - 1];
   g.nrows = L[nd - 2];
-  if (Lf > PLQ_HALO || Lf < 2) return false;
+  if (Lf > PLQ_ROW || Lf < 2) return false;
   const uint64_t two32 = 1ull << 32;
   if ((uint64_t)V * 32u >= two32) return false;  // 32-bit byte offsets in a plane
   double best = 0.0;
@@ -214,6 +217,10 @@ template <typename T_> struct PlqSU2 {
   using link = quat<T>;
   static constexpr int NM = 3;
   using V = pv3<T>;
+  // P' = P - DF coef ep Im(U K); a plaquette adds RP re to the sum of ReTr(U K) over its links
+  static constexpr double DF = 2.0, RP = 8.0;
+  // LDS bytes of ND links, an odd multiple of 16
+  static constexpr int lrec(int nd) { return (nd * (int)sizeof(link) / 16 | 1) * 16; }
   // B, C: whether the b / c term is wanted; RE: re += w ReTr(P) / 2
   template <bool B, bool C, bool RE>
   __device__ static void plane(const link &a, const link &b, const link &c, const link &d, V &v0,
@@ -232,10 +239,106 @@ template <typename T_> struct PlqSU2 {
   }
 };
 
+// sin and cos of t = q pi/2 + r, |r| <= pi/4 (pi/2 in two parts, the first of
+// 33 bits, so that q times it is exact for the q < 2^17 that occur), by Taylor
+// series in r^2 to the eighth power (remainders below 1e-18)
+__device__ __forceinline__ void plq_series(double y, double &c, double &s) {
+  double t = fma(y, 1.0 / 20922789888000.0, -1.0 / 87178291200.0);
+  double u = fma(y, 1.0 / 355687428096000.0, -1.0 / 1307674368000.0);
+  t = fma(y, t, 1.0 / 479001600);
+  u = fma(y, u, 1.0 / 6227020800.0);
+  t = fma(y, t, -1.0 / 3628800);
+  u = fma(y, u, -1.0 / 39916800);
+  t = fma(y, t, 1.0 / 40320);
+  u = fma(y, u, 1.0 / 362880);
+  t = fma(y, t, -1.0 / 720);
+  u = fma(y, u, -1.0 / 5040);
+  t = fma(y, t, 1.0 / 24);
+  u = fma(y, u, 1.0 / 120);
+  t = fma(y, t, -0.5);
+  u = fma(y, u, -1.0 / 6);
+  c = fma(y, t, 1.0);
+  s = fma(y, u, 1.0);
+}
+__device__ __forceinline__ double plq_reduce(double a, int &j) {
+  if (fabs(a) > 1e5) a = fmod(a, 6.283185307179586477);
+  const double q = rint(a * 0.6366197723675813431);
+  j = (int)q;
+  return fma(-q, 6.07710050650619224932e-11, fma(-q, 1.57079632673412561417, a));
+}
+__device__ __forceinline__ void plq_quadrant(int j, double &c, double &s) {
+  const double sn = (j & 1) ? c : s, cs = (j & 1) ? s : c;
+  c = ((j + 1) & 2) ? -cs : cs;
+  s = (j & 2) ? -sn : sn;
+}
+
+// U(1): the links of a plaquette are phases, and every link's term is the sine of
+// their sum with its sign; FP32 links are added in FP64
+template <typename T_> struct PlqU1 {
+  using T = T_;
+  using link = T;
+  static constexpr int NM = 1;
+  struct V {
+    T k[1];
+  };
+  static constexpr double DF = 1.0, RP = 4.0;
+  static constexpr int lrec(int nd) { return (nd | 1) * (int)sizeof(T); }
+  template <bool RE> __device__ static T sine(T a, T b, T c, T d, double &co) {
+    const double th = ((double(a) + double(b)) - double(c)) - double(d);
+    if constexpr (sizeof(T) == 4) {
+      // a reduced argument rounded once, |r| <= pi: the FP32 functions' fast range
+      const float r = (float)fma(-rint(th * 0.15915494309189533577), 6.283185307179586477, th);
+      if (RE) co = cos(th);
+      return sinf(r);
+    } else {
+      int j;
+      const double r = plq_reduce(th, j);
+      double cs, sn;
+      plq_series(r * r, cs, sn);
+      sn *= r;
+      plq_quadrant(j, cs, sn);
+      if (RE) co = cs;
+      return sn;
+    }
+  }
+  template <bool B, bool C, bool RE>
+  __device__ static void plane(link a, link b, link c, link d, V &v0, V &vb, V &vc, double w,
+                               double &re) {
+    double co = 0.0;
+    const T s = sine<RE>(a, b, c, d, co);
+    if (RE) re = fma(w, co, re);
+    v0.k[0] = s;
+    if (B) vb.k[0] = s;
+    if (C) vc.k[0] = -s;
+  }
+  __device__ static V lowb(link a, link b, link c, link d) {
+    double co;
+    return V{{sine<false>(a, b, c, d, co)}};
+  }
+  __device__ static V lowc(link a, link b, link c, link d) {
+    double co;
+    return V{{-sine<false>(a, b, c, d, co)}};
+  }
+};
+
 // ------------------------------------------------------------------- memory --
 __device__ __forceinline__ void plq_barrier() {
   // LDS writes done, then the barrier; global loads may stay in flight
   asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+
+// fields of phases
+template <typename T, typename = std::enable_if_t<std::is_floating_point<T>::value>>
+__device__ __forceinline__ T *fld_add(T *p, size_t k) {
+  return p + k;
+}
+template <typename T, typename = std::enable_if_t<std::is_floating_point<T>::value>>
+__device__ __forceinline__ const T *fld_add(const T *p, size_t k) {
+  return p + k;
+}
+template <typename T, typename = std::enable_if_t<std::is_floating_point<T>::value>>
+__device__ __forceinline__ T ldq(const T *__restrict__ p, uint32_t i) {
+  return ldo(p, i);
 }
 
 // The exchange in LDS: one record per thread (and of a halo row) with the nd
@@ -243,9 +346,6 @@ __device__ __forceinline__ void plq_barrier() {
 // are immediates of the LDS instructions, so a thread needs one address per
 // neighbour; records are odd multiples of 16 B (links) or 8 B apart modulo the
 // banks, so the lanes of an access spread over them.
-template <class G, int ND> constexpr int plq_lrec() {
-  return (ND * (int)sizeof(typename G::link) / 16 | 1) * 16;
-}
 template <class G, int ND> constexpr int plq_vrec() {
   return (2 * (ND - 1) * G::NM | 1) * (int)sizeof(typename G::T);
 }
@@ -266,73 +366,59 @@ __device__ __forceinline__ void plq_get(const char *rec, int k, quat<float> &q) 
   const su2_f4 a = ((const su2_f4 *)rec)[k];
   q = quat<float>{a.x, a.y, a.z, a.w};
 }
-template <typename T> __device__ __forceinline__ void plq_putv(char *rec, int k, const pv3<T> &v) {
-  T *p = (T *)rec + 3 * k;
-  p[0] = v.k[0];
-  p[1] = v.k[1];
-  p[2] = v.k[2];
+template <typename T> __device__ __forceinline__ void plq_put(char *rec, int k, const T &q) {
+  ((T *)rec)[k] = q;
 }
-template <typename T>
-__device__ __forceinline__ void plq_getv(const char *rec, int k, pv3<T> &v) {
-  const T *p = (const T *)rec + 3 * k;
-  v.k[0] = p[0];
-  v.k[1] = p[1];
-  v.k[2] = p[2];
+template <typename T> __device__ __forceinline__ void plq_get(const char *rec, int k, T &q) {
+  q = ((const T *)rec)[k];
+}
+template <class G>
+__device__ __forceinline__ void plq_putv(char *rec, int k, const typename G::V &v) {
+  typename G::T *p = (typename G::T *)rec + G::NM * k;
+#pragma unroll
+  for (int i = 0; i < G::NM; ++i) p[i] = v.k[i];
+}
+template <class G>
+__device__ __forceinline__ void plq_getv(const char *rec, int k, typename G::V &v) {
+  const typename G::T *p = (const typename G::T *)rec + G::NM * k;
+#pragma unroll
+  for (int i = 0; i < G::NM; ++i) v.k[i] = p[i];
 }
 template <class G, int ND> size_t plq_lds(const PlqGeo &g) {
   const size_t nt = plq_threads(g);
-  return (nt + g.L[g.nd - 1]) * plq_lrec<G, ND>() + nt * plq_vrec<G, ND>();
+  return (nt + g.L[g.nd - 1]) * G::lrec(ND) + nt * plq_vrec<G, ND>();
 }
 
 // the values are complete here: keeps the compiler from sinking their arithmetic
 // past later loads, which would hold its operands in registers
-template <typename T> __device__ __forceinline__ void plq_pin(T (&v)[3]) {
-  asm volatile("" : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]));
+template <typename T, int N> __device__ __forceinline__ void plq_pin(T (&v)[N]) {
+#pragma unroll
+  for (int k = 0; k < N; ++k) asm volatile("" : "+v"(v[k]));
 }
 
 // acc += w v
-template <typename V> __device__ __forceinline__ void plq_add(double (&acc)[3], double w, const V &v) {
+template <int N, typename V>
+__device__ __forceinline__ void plq_add(double (&acc)[N], double w, const V &v) {
 #pragma unroll
-  for (int k = 0; k < 3; ++k) acc[k] = fma(w, double(v.k[k]), acc[k]);
+  for (int k = 0; k < N; ++k) acc[k] = fma(w, double(v.k[k]), acc[k]);
 }
 
-// cos a and sin(a)/a of the FP64 update for x = a^2: Taylor series in y to y^8
-// (remainders y^9 / 18! <= 1.6e-16 and y^9 / 19! for y <= 1, at most an ulp
-// with the Horner roundings), y = x where x <= 1; beyond that y = r^2 with
-// a = q pi/2 + r, |r| <= pi/4 (pi/2 in two parts, the first of 33 bits, so that
-// q times it is exact for the q < 2^17 that occur).
+// cos a and sin(a)/a of the FP64 update for x = a^2: the series in x where
+// x <= 1 (remainders x^9 / 18! <= 1.6e-16 and x^9 / 19!), beyond that in the
+// square of the reduced angle
 __device__ __forceinline__ void cos_sinc_fp64(double x, double &c, double &s) {
-  double y = x, r = 0.0, q = 0.0;
+  double y = x, r = 0.0;
+  int j = 0;
   const bool big = !(x <= 1.0);
   if (big) {
-    double al = sqrt(x);
-    if (al > 1e5) al = fmod(al, 6.283185307179586477);
-    q = rint(al * 0.6366197723675813431);
-    r = fma(-q, 6.07710050650619224932e-11, fma(-q, 1.57079632673412561417, al));
+    r = plq_reduce(sqrt(x), j);
     y = r * r;
   }
-  double t = fma(y, 1.0 / 20922789888000.0, -1.0 / 87178291200.0);
-  double u = fma(y, 1.0 / 355687428096000.0, -1.0 / 1307674368000.0);
-  t = fma(y, t, 1.0 / 479001600);
-  u = fma(y, u, 1.0 / 6227020800.0);
-  t = fma(y, t, -1.0 / 3628800);
-  u = fma(y, u, -1.0 / 39916800);
-  t = fma(y, t, 1.0 / 40320);
-  u = fma(y, u, 1.0 / 362880);
-  t = fma(y, t, -1.0 / 720);
-  u = fma(y, u, -1.0 / 5040);
-  t = fma(y, t, 1.0 / 24);
-  u = fma(y, u, 1.0 / 120);
-  t = fma(y, t, -0.5);
-  u = fma(y, u, -1.0 / 6);
-  c = fma(y, t, 1.0);
-  s = fma(y, u, 1.0);
+  plq_series(y, c, s);
   if (big) {
-    const int j = (int)q;
-    const double sr = r * s;
-    const double sn = (j & 1) ? c : sr, cs = (j & 1) ? sr : c;
-    c = ((j + 1) & 2) ? -cs : cs;
-    s = ((j & 2) ? -sn : sn) / sqrt(x);
+    s *= r;
+    plq_quadrant(j, c, s);
+    s = s / sqrt(x);
   }
 }
 
@@ -342,21 +428,23 @@ template <typename T> __device__ __forceinline__ uint32_t plq_off(uint32_t V, in
   return (i + (uint32_t)k * V) * (uint32_t)sizeof(T);
 }
 
-// momentum and link update of one link from G = Im(U K):
-// P' = P - 2 coef ep G rounded once, U' = exp(eu P') U
-template <typename T, bool W, int NT, class UO>
-__device__ __forceinline__ void plq_update(const quat<T> &u, const double (&G)[3],
-                                           const T (&pi)[3], T (&pn)[3], T *Pw, uint32_t V, UO Uo,
-                                           uint32_t s, const FusedCoef &c) {
-  const double f = 2.0 * c.coef * c.ep;
+// momentum and link update of one link from F = Im(U K):
+// P' = P - DF coef ep F rounded once, U' = exp(eu P') U
+template <class G, bool W, int NT, class UO, typename T = typename G::T>
+__device__ __forceinline__ void plq_update(const typename G::link &u, const double (&F)[G::NM],
+                                           const T (&pi)[G::NM], T (&pn)[G::NM], T *Pw,
+                                           uint32_t V, UO Uo, uint32_t s, const FusedCoef &c) {
+  const double f = G::DF * c.coef * c.ep;
 #pragma unroll
-  for (int k = 0; k < 3; ++k) {
-    pn[k] = T(fma(-f, G[k], double(pi[k])));
+  for (int k = 0; k < G::NM; ++k) {
+    pn[k] = T(fma(-f, F[k], double(pi[k])));
     T *q = (T *)((char *)Pw + plq_off<T>(V, k, s));
     if (NT) __builtin_nontemporal_store(pn[k], q);
     else *q = pn[k];
   }
-  if constexpr (W) {
+  if constexpr (W && G::NM == 1) {
+    sto_h<NT>(Uo, s, T(fma(c.eu, double(pn[0]), double(u))));
+  } else if constexpr (W) {
     const double e0 = c.eu * double(pn[0]), e1 = c.eu * double(pn[1]), e2 = c.eu * double(pn[2]);
     const double x = fma(e0, e0, fma(e1, e1, e2 * e2));
     double cs, sn;
@@ -377,18 +465,19 @@ __device__ __forceinline__ void plq_update(const quat<T> &u, const double (&G)[3
 
 // ------------------------------------------------------------------ the step --
 // W: write the new links (false: momenta alone); ACC: block partials of
-// |P_in|^2, ReTr(U K) and |P_out|^2.  pin / pout may be the same field.
+// |P_in|^2, ReTr(U K) (FP64; 0 in FP32) and |P_out|^2.  pin / pout may be the same field.
 // flags: F_PZERO (momenta read as zero), F_RESTORE; w_t / w_s weight the planes
 // (1 where isotropic: fma with 1 is the plain sum).  GEN: the momenta are drawn
 // (Philox counter of k_momenta_philox) instead of loaded.  NT: 0 ordinary
 // accesses, 2 non-temporal stores and momentum loads.
 template <class G, int ND, bool W, bool ACC, bool GEN, int NT, class UI, class UO>
-__global__ __launch_bounds__(PLQ_NT, sizeof(typename G::T) == 8 ? 2 : 3) void k_md_plq(
+__global__ __launch_bounds__(PLQ_NT, G::NM == 1 ? 4 : sizeof(typename G::T) == 8 ? 2 : 3) void k_md_plq(
     UI Uin, UO Uout, const typename G::T *Pin, typename G::T *Pout, PlqGeo g, FusedCoef c,
     double *__restrict__ partials, int pstride) {
   using T = typename G::T;
   using link = typename G::link;
   using Vc = typename G::V;
+  constexpr int NM = G::NM;
   extern __shared__ __align__(16) char smem[];
   const int nt = (int)blockDim.x, tid = (int)threadIdx.x;
   constexpr int R = ND - 2, Z = ND - 1;              // row and fastest direction
@@ -397,7 +486,7 @@ __global__ __launch_bounds__(PLQ_NT, sizeof(typename G::T) == 8 ? 2 : 3) void k_
   const size_t V = (size_t)g.V;
   // LDS records: own, of the row above (or the halo's), of x+z; the terms' of
   // own, of the row below, of x-z
-  constexpr int LREC = plq_lrec<G, ND>(), VREC = plq_vrec<G, ND>();
+  constexpr int LREC = G::lrec(ND), VREC = plq_vrec<G, ND>();
   char *const lv0 = smem + (nt + g.L[Z]) * LREC;
   char *const lown = smem + tid * LREC, *const lrow = smem + f.lur * LREC,
              *const lz = smem + f.luz * LREC;
@@ -409,6 +498,8 @@ __global__ __launch_bounds__(PLQ_NT, sizeof(typename G::T) == 8 ? 2 : 3) void k_
   const bool rin = f.rin, din = f.ldr >= 0;
   const bool edge = __builtin_amdgcn_readfirstlane((int)(__ballot(!din) != 0)) != 0;
   const double wt = c.w_t, ws = c.w_s;
+  // the action partial is the FP64 form's (FP32 takes the plaquette sum)
+  constexpr bool RE = ACC && sizeof(T) == 8;
   double sums[3] = {0.0, 0.0, 0.0};
   double re = 0.0;
 
@@ -431,7 +522,7 @@ __global__ __launch_bounds__(PLQ_NT, sizeof(typename G::T) == 8 ? 2 : 3) void k_
   }
   for (int t = f.t0; t < f.t1; ++t) {
     const int ut = up_t(t);
-    double acc[ND][3];
+    double acc[ND][NM];
     link nx[ND], ux[ND], xlt;
     {
       // every load of the slice but the momenta's, in the order of use
@@ -469,8 +560,9 @@ __global__ __launch_bounds__(PLQ_NT, sizeof(typename G::T) == 8 ? 2 : 3) void k_
 #pragma unroll
       for (int i = 1; i < ND; ++i)
 #pragma unroll
-        for (int k = 0; k < 3; ++k) acc[i][k] = wt * double(carry[i].k[k]);
-      acc[0][0] = acc[0][1] = acc[0][2] = 0.0;
+        for (int k = 0; k < NM; ++k) acc[i][k] = wt * double(carry[i].k[k]);
+#pragma unroll
+      for (int k = 0; k < NM; ++k) acc[0][k] = 0.0;
       if constexpr (X4) {
         plq_add(acc[0], wt, G::lowc(lx[0], xlt, own[0], xl));        // (t, x) at x-1
         plq_add(acc[2], ws, G::lowb(xl, own[2], lxu[2], lx[2]));     // (x, y)
@@ -481,7 +573,7 @@ __global__ __launch_bounds__(PLQ_NT, sizeof(typename G::T) == 8 ? 2 : 3) void k_
       for (int m = 0; m < ND; ++m) plq_pin(acc[m]);
     }
     plq_barrier();
-    T pi[ND][3];
+    T pi[ND][NM];
     link eR, e0, eRt, eZ, eRz, eX, eRx;
     {
       Vc v0, vb, vc;
@@ -490,47 +582,47 @@ __global__ __launch_bounds__(PLQ_NT, sizeof(typename G::T) == 8 ? 2 : 3) void k_
       // (r, z): b term to U_z(x+r), c term to U_r(x+z)
       plq_get(lrow, Z, p);
       plq_get(lz, R, q);
-      G::template plane<true, true, ACC>(own[R], p, q, own[Z], v0, vb, vc, 1.0, res);
+      G::template plane<true, true, RE>(own[R], p, q, own[Z], v0, vb, vc, 1.0, res);
       plq_add(acc[R], ws, v0);
       plq_add(acc[Z], -ws, v0);
-      plq_putv(vown, ND - 2, vb);
-      plq_putv(vown, 2 * (ND - 1) - 1, vc);
+      plq_putv<G>(vown, ND - 2, vb);
+      plq_putv<G>(vown, 2 * (ND - 1) - 1, vc);
       __builtin_amdgcn_sched_barrier(0);
       // (t, r): c term to U_t(x+r); (t, z): to U_t(x+z)
       plq_get(lrow, 0, q);
-      G::template plane<true, true, ACC>(own[0], nx[R], q, own[R], v0, vb, vc, 1.0, ret);
+      G::template plane<true, true, RE>(own[0], nx[R], q, own[R], v0, vb, vc, 1.0, ret);
       plq_add(acc[0], wt, v0);
       plq_add(acc[R], -wt, v0);
       carry[R] = vb;
-      plq_putv(vown, 0, vc);
+      plq_putv<G>(vown, 0, vc);
       __builtin_amdgcn_sched_barrier(0);
       plq_get(lz, 0, q);
-      G::template plane<true, true, ACC>(own[0], nx[Z], q, own[Z], v0, vb, vc, 1.0, ret);
+      G::template plane<true, true, RE>(own[0], nx[Z], q, own[Z], v0, vb, vc, 1.0, ret);
       plq_add(acc[0], wt, v0);
       plq_add(acc[Z], -wt, v0);
       carry[Z] = vb;
-      plq_putv(vown, ND - 1, vc);
+      plq_putv<G>(vown, ND - 1, vc);
       __builtin_amdgcn_sched_barrier(0);
       if constexpr (X4) {
         plq_get(lrow, 1, q);
-        G::template plane<false, true, ACC>(own[1], ux[2], q, own[2], v0, vb, vc, 1.0, res);
+        G::template plane<false, true, RE>(own[1], ux[2], q, own[2], v0, vb, vc, 1.0, res);
         plq_add(acc[1], ws, v0);
         plq_add(acc[2], -ws, v0);
-        plq_putv(vown, 1, vc);
+        plq_putv<G>(vown, 1, vc);
         __builtin_amdgcn_sched_barrier(0);
         plq_get(lz, 1, q);
-        G::template plane<false, true, ACC>(own[1], ux[3], q, own[3], v0, vb, vc, 1.0, res);
+        G::template plane<false, true, RE>(own[1], ux[3], q, own[3], v0, vb, vc, 1.0, res);
         plq_add(acc[1], ws, v0);
         plq_add(acc[3], -ws, v0);
-        plq_putv(vown, ND, vc);
+        plq_putv<G>(vown, ND, vc);
         __builtin_amdgcn_sched_barrier(0);
-        G::template plane<true, false, ACC>(own[0], nx[1], ux[0], own[1], v0, vb, vc, 1.0, ret);
+        G::template plane<true, false, RE>(own[0], nx[1], ux[0], own[1], v0, vb, vc, 1.0, ret);
         plq_add(acc[0], wt, v0);
         plq_add(acc[1], -wt, v0);
         carry[1] = vb;
         __builtin_amdgcn_sched_barrier(0);
       }
-      if (ACC) {
+      if (RE) {
         if (f.active) re += fma(wt, ret, ws * res);
         asm volatile("" : "+v"(re));
       }
@@ -546,19 +638,19 @@ __global__ __launch_bounds__(PLQ_NT, sizeof(typename G::T) == 8 ? 2 : 3) void k_
           philox_normals4<T>((uint32_t)(s * ND + m), (uint32_t)(c.gtraj & 0xffffffffu),
                              (uint32_t)(c.gtraj >> 32), c.gseed, z);
 #pragma unroll
-          for (int k = 0; k < 3; ++k) pi[m][k] = z[k];
+          for (int k = 0; k < NM; ++k) pi[m][k] = z[k];
         }
       } else if (c.flags & F_PZERO) {
 #pragma unroll
         for (int m = 0; m < ND; ++m)
 #pragma unroll
-          for (int k = 0; k < 3; ++k) pi[m][k] = T(0);
+          for (int k = 0; k < NM; ++k) pi[m][k] = T(0);
       } else {
 #pragma unroll
         for (int m = 0; m < ND; ++m) {
-          const char *p = (const char *)(Pin + (size_t)(m * 3) * V);
+          const char *p = (const char *)(Pin + (size_t)(m * NM) * V);
 #pragma unroll
-          for (int k = 0; k < 3; ++k) {
+          for (int k = 0; k < NM; ++k) {
             const T *q = (const T *)(p + plq_off<T>((uint32_t)g.V, k, (uint32_t)s));
             if constexpr (NT == 2) pi[m][k] = __builtin_nontemporal_load(q);
             else pi[m][k] = *q;
@@ -584,23 +676,23 @@ __global__ __launch_bounds__(PLQ_NT, sizeof(typename G::T) == 8 ? 2 : 3) void k_
     {
       Vc v;
       // from x-z: U_t, U_x (d = 4), U_r
-      plq_getv(vz, ND - 1, v);
+      plq_getv<G>(vz, ND - 1, v);
       plq_add(acc[0], wt, v);
       if constexpr (X4) {
-        plq_getv(vz, ND, v);
+        plq_getv<G>(vz, ND, v);
         plq_add(acc[1], ws, v);
       }
-      plq_getv(vz, 2 * (ND - 1) - 1, v);
+      plq_getv<G>(vz, 2 * (ND - 1) - 1, v);
       plq_add(acc[R], ws, v);
       if (din) {
         // from x-r: U_t, U_x (d = 4), U_z
-        plq_getv(vrow, 0, v);
+        plq_getv<G>(vrow, 0, v);
         plq_add(acc[0], wt, v);
         if constexpr (X4) {
-          plq_getv(vrow, 1, v);
+          plq_getv<G>(vrow, 1, v);
           plq_add(acc[1], ws, v);
         }
-        plq_getv(vrow, ND - 2, v);
+        plq_getv<G>(vrow, ND - 2, v);
         plq_add(acc[Z], ws, v);
       }
       if (edge) {
@@ -615,13 +707,16 @@ __global__ __launch_bounds__(PLQ_NT, sizeof(typename G::T) == 8 ? 2 : 3) void k_
       if (f.active) {
 #pragma unroll
         for (int m = 0; m < ND; ++m) {
-          T pn[3];
-          plq_update<T, W, NT>(own[m], acc[m], pi[m], pn,
-                               Pout + (size_t)(m * 3) * V, (uint32_t)g.V,
+          T pn[NM];
+          plq_update<G, W, NT>(own[m], acc[m], pi[m], pn,
+                               Pout + (size_t)(m * NM) * V, (uint32_t)g.V,
                                fld_add(Uout, (size_t)m * V), (uint32_t)s, c);
           if (ACC) {
-            sums[0] += sq3(pi[m][0], pi[m][1], pi[m][2]);
-            sums[2] += sq3(pn[0], pn[1], pn[2]);
+#pragma unroll
+            for (int k = 0; k < NM; ++k) {
+              sums[0] = fma(double(pi[m][k]), double(pi[m][k]), sums[0]);
+              sums[2] = fma(double(pn[k]), double(pn[k]), sums[2]);
+            }
           }
         }
       }
@@ -635,7 +730,7 @@ __global__ __launch_bounds__(PLQ_NT, sizeof(typename G::T) == 8 ? 2 : 3) void k_
   }
   if (ACC) {
     // ReTr(U K) of every link: a plaquette's 2 Re(P) once for each of its four
-    sums[1] = 8.0 * re;
+    sums[1] = G::RP * re;
     __syncthreads();
     double *l3 = (double *)smem;
     const int lane = tid & 63, wv = tid >> 6, nw = nt >> 6;

@@ -7,25 +7,27 @@ namespace {
 
 constexpr int CUS = 256;  // MI355X
 
-// resident blocks on a CU: registers leave room for 8 waves (FP64, 2 per SIMD)
-// or 12 (FP32), LDS for 160 KB
-template <class G, int ND> int plq_percu(const PlqGeo &g) {
-  const int waves = (int)plq_threads(g) / 64, lds = (int)plq_lds<G, ND>(g);
-  return std::max(1, std::min((sizeof(typename G::T) == 8 ? 8 : 12) / waves, 160 * 1024 / lds));
+// resident blocks on a CU: registers leave room for 8 waves (SU(2) FP64, 2 per
+// SIMD), 12 (SU(2) FP32) or 16 (U(1)), LDS for 160 KB
+template <class G> int plq_percu(const PlqGeo &g) {
+  const int waves = (int)plq_threads(g) / 64;
+  const int lds = (int)(g.nd == 4 ? plq_lds<G, 4>(g) : plq_lds<G, 3>(g));
+  const int fit = G::NM == 1 ? 16 : sizeof(typename G::T) == 8 ? 8 : 12;
+  return std::max(1, std::min(fit / waves, 160 * 1024 / lds));
 }
 
 // The layout, or false where the staple steps are taken instead.  Below 32768
 // (FP64) and 98304 sites (FP32) those are as fast or faster: a launch is bound by
 // its chain of memory round trips, of which this step has two more (FP64 step
 // with events, this / staples: 12^4 10.2 / 9.8, 16^4 12.3 / 13.1, d = 3 32^3 8.5 /
-// 8.7 us; FP32: 16^4 10.5 / 9.7, 20^4 15.8 / 16.2, d = 3 21 59 79 10.1 / 10.3 us).
+// 8.7 us; FP32: 16^4 10.5 / 9.7, 20^4 15.8 / 16.2, d = 3 21 59 79 10.1 / 10.3 us;
+// U(1) FP64 12^4 8.9 / 8.1, 16^4 9.1 / 11.1, d = 3 32^3 6.8 / 7.1 us, FP32 16^4 8.1 /
+// 7.7, 20 18 15 27 10.2 / 11.4 us).
 bool plq_geo_for(int group, int prec, const Geo &geo, PlqGeo &g) {
-  if (group != 1 || geo.V < (prec == 0 ? 32768 : 98304)) return false;
+  if (geo.V < (prec == 0 ? 32768 : 98304)) return false;
   if (!make_plq_rows(geo.L, geo.nd, geo.V, g)) return false;
-  const int percu = prec == 0 ? (geo.nd == 4 ? plq_percu<PlqSU2<double>, 4>(g)
-                                             : plq_percu<PlqSU2<double>, 3>(g))
-                              : (geo.nd == 4 ? plq_percu<PlqSU2<float>, 4>(g)
-                                             : plq_percu<PlqSU2<float>, 3>(g));
+  const int percu = group == 1 ? (prec == 0 ? plq_percu<PlqSU2<double>>(g) : plq_percu<PlqSU2<float>>(g))
+                               : (prec == 0 ? plq_percu<PlqU1<double>>(g) : plq_percu<PlqU1<float>>(g));
   return make_plq_chunks(percu, CUS, g);
 }
 
@@ -80,9 +82,10 @@ bool launch_plq(int group, int prec, const FusedLaunch &L, hipStream_t st) {
   // momenta exceed the 256 MB Infinity Cache: FP64 32^4 (369 MB) 106.9 against
   // 109.4 us with the stores alone and 124 with neither, FP32 48^4 284.9 /
   // 293.5 / 315; below, FP64 24^4 (117 MB) 43.5 with them and 38.8 without
-  const double fields = (double)L.geo.nd * L.geo.V * (prec == 0 ? 88.0 : 44.0);
+  const double fields =
+      (double)L.geo.nd * L.geo.V * (group == 1 ? 11.0 : 3.0) * (prec == 0 ? 8.0 : 4.0);
   const bool nt = fields > 256.0 * 1024 * 1024;
-  if (prec == 0 && L.geo.nd == 4) {
+  if (group == 1 && prec == 0 && L.geo.nd == 4) {
     const size_t nl = 4 * (size_t)L.geo.V;
     const su2_d2 *ia = (const su2_d2 *)L.Uin;
     su2_d2 *oa = (su2_d2 *)L.Uout;
@@ -95,11 +98,19 @@ bool launch_plq(int group, int prec, const FusedLaunch &L, hipStream_t st) {
     return true;
   }
   if (L.in_half || L.out_half) return false;
-#define SU2_PLQ(T, ND) \
-  go_wa<PlqSU2<T>, ND>((const quat<T> *)L.Uin, (quat<T> *)L.Uout, L, g, nt, st)
-  if (prec == 0) SU2_PLQ(double, 3);
-  else if (L.geo.nd == 4) SU2_PLQ(float, 4);
-  else SU2_PLQ(float, 3);
+#define SU2_PLQ(G, ND)                                                                    \
+  go_wa<G, ND>((const typename G::link *)L.Uin, (typename G::link *)L.Uout, L, g, nt, st)
+  if (group == 1) {
+    if (prec == 0) SU2_PLQ(PlqSU2<double>, 3);
+    else if (L.geo.nd == 4) SU2_PLQ(PlqSU2<float>, 4);
+    else SU2_PLQ(PlqSU2<float>, 3);
+  } else if (L.geo.nd == 4) {
+    if (prec == 0) SU2_PLQ(PlqU1<double>, 4);
+    else SU2_PLQ(PlqU1<float>, 4);
+  } else {
+    if (prec == 0) SU2_PLQ(PlqU1<double>, 3);
+    else SU2_PLQ(PlqU1<float>, 3);
+  }
 #undef SU2_PLQ
   return true;
 }

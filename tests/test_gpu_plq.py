@@ -7,7 +7,7 @@ half-field layout ((16, 8, 8, 32), 3-volume a multiple of 256).
 Tolerances: five force and four link sweeps with O(1) operands add some 20
 roundings per sweep; FP64 20 * 9 * 2^-53 = 2e-14, taken as 1e-12 as for one
 sweep elsewhere; FP32 (links and momenta rounded to 2^-24 per sweep) 20 * 9 *
-2^-24 = 1.1e-5."""
+2^-24 = 1.1e-5.  U(1) phases go up to 4 rather than 1: four times that."""
 import numpy as np
 import pytest
 
@@ -27,44 +27,47 @@ CASES = [  # Lx, Ly, Lz, Lt, nd, xi
 
 @pytest.mark.parametrize("case", CASES)
 @pytest.mark.parametrize("prec", [0, 1])
-def test_trajectory_matches_oracle(oracle, case, prec):
+@pytest.mark.parametrize("group", [1, 0])
+def test_trajectory_matches_oracle(oracle, case, prec, group):
     *dims, xi = case
     dims = tuple(dims)
     if prec == 1 and dims[0] * dims[1] * dims[2] * dims[3] < 98304:
         # the FP32 form takes the step from 98304 sites
         dims = dims[:3] + (-(-98304 // (dims[0] * dims[1] * dims[2])),) + dims[4:]
-    U0 = oracle.hotstart(1, dims, SEED, 0.4)
-    P0 = oracle.initnormal(1, dims, SEED + 1)
+    U0 = oracle.hotstart(group, dims, SEED, 0.4)
+    P0 = oracle.initnormal(group, dims, SEED + 1)
     if prec == 1:
         U0 = U0.astype(np.float32).astype(np.float64)
         P0 = P0.astype(np.float32).astype(np.float64)
-    U_ref, P_ref = oracle.integrate(1, dims, U0, P0.copy(), 2.4, S.OMF2, 2, tau=0.2, xi=xi)
-    with S.Lattice(S.SU2, dims, 2.4, xi=xi, precision=prec) as lat:
+    U_ref, P_ref = oracle.integrate(group, dims, U0, P0.copy(), 2.4, S.OMF2, 2, tau=0.2, xi=xi)
+    with S.Lattice(group, dims, 2.4, xi=xi, precision=prec) as lat:
         lat.set_links(U0)
         r = lat.md_trajectory(P0, S.OMF2, 2, tau=0.2)
         lat.md_finish(True)
         U, P = lat.get_links(), lat.get_momenta()
-    assert np.abs(U - U_ref).max() < TOL[prec]
-    assert np.abs(P - P_ref).max() < 10 * TOL[prec]  # momenta up to ~5, forces up to ~10
+    tol = TOL[prec] * (1 if group == 1 else 4)
+    assert np.abs(U - U_ref).max() < tol
+    assert np.abs(P - P_ref).max() < 10 * tol  # momenta up to ~5, forces up to ~10
     # the step's own partial sums: kinetic energies and the start's action
-    assert r["kin_old"] == pytest.approx(oracle.kinetic(1, dims, P0, compensated=True), rel=1e-13)
-    assert r["kin_new"] == pytest.approx(oracle.kinetic(1, dims, P, compensated=True), rel=1e-13)
+    assert r["kin_old"] == pytest.approx(oracle.kinetic(group, dims, P0, compensated=True), rel=1e-13)
+    assert r["kin_new"] == pytest.approx(oracle.kinetic(group, dims, P, compensated=True), rel=1e-13)
     assert r["gauge_old"] == pytest.approx(
-        oracle.action(1, dims, U0, 2.4, xi=xi, compensated=True), rel=1e-13)
+        oracle.action(group, dims, U0, 2.4, xi=xi, compensated=True), rel=1e-13)
 
 
 @pytest.mark.parametrize("dims", [(16, 8, 8, 32, 4), (5, 9, 61, 13, 4), (59, 21, 1, 79, 3)])
-def test_momentum_only_and_zero_momentum_steps(oracle, dims):
+@pytest.mark.parametrize("group", [1, 0])
+def test_momentum_only_and_zero_momentum_steps(oracle, dims, group):
     """The force alone (derivative), and the Runge-Kutta stages, whose first
     reads its momenta as zero (flat-gradient_flow.hh:17-50)."""
-    U0 = oracle.hotstart(1, dims, SEED, 0.4)
-    with S.Lattice(S.SU2, dims, 2.4) as lat:
+    U0 = oracle.hotstart(group, dims, SEED, 0.4)
+    with S.Lattice(group, dims, 2.4) as lat:
         lat.set_links(U0)
         D = lat.derivative(1.0)
         lat.runge_kutta(0.01)
         W = lat.get_links()
-    assert np.abs(D - oracle.derivative(1, dims, U0, 2.4)).max() < 1e-12
-    assert np.abs(W - oracle.runge_kutta(1, dims, U0, 2.4, 0.01)).max() < 1e-12
+    assert np.abs(D - oracle.derivative(group, dims, U0, 2.4)).max() < 1e-12
+    assert np.abs(W - oracle.runge_kutta(group, dims, U0, 2.4, 0.01)).max() < 1e-12
 
 
 def test_update_angles_beyond_the_series(oracle):

@@ -16,7 +16,7 @@ CASES = [
     (4, (8, 4, 32, 32), 3), (4, (27, 20, 18, 15), 3), (4, (12, 6, 24, 24), 3),
     (4, (7, 3, 48, 48), 1), (4, (4, 4, 4, 4), 3), (4, (2, 2, 2, 2), 3),
     (4, (1, 1, 1, 2), 3), (4, (3, 1, 2, 64), 1), (4, (5, 2, 40, 40), 2),
-    (4, (16, 3, 5, 3), 1), (4, (9, 2, 7, 61), 3), (3, (21, 16, 16, 1), 3),
+    (4, (5, 2, 3, 128), 2), (4, (16, 3, 5, 3), 1), (4, (9, 2, 7, 61), 3), (3, (21, 16, 16, 1), 3),
     (3, (79, 21, 59, 1), 8), (3, (3, 2, 64, 1), 4), (3, (8, 5, 3, 1), 8),
 ]
 
@@ -41,7 +41,7 @@ def test_every_site_once_with_its_neighbours(check, nd, ext, slots):
 
 
 def test_not_applicable_geometries(check):
-    # a row longer than the halo, a row of one site
-    for ext in ((4, 4, 4, 65), (4, 4, 4, 1)):
+    # a row longer than the longest taken, a row of one site
+    for ext in ((4, 4, 4, 129), (4, 4, 4, 1)):
         out = subprocess.run([check, "4", *map(str, ext), "2"], capture_output=True, text=True)
         assert out.returncode == 0 and out.stdout.startswith("not applicable")
