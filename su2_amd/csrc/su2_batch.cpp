@@ -265,8 +265,6 @@ int enqueue(B *b, bool devmom, Rec *rec = nullptr) {
   fin();
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return bfail(SU2GPU_EHIP, "batch launch: %s", hipGetErrorString(e));
-  BH(hipMemcpyAsync(b->hsums, b->dsums, (size_t)n * 2 * NSUM * sizeof(double),
-                    hipMemcpyDeviceToHost, b->stream));
   return SU2GPU_OK;
 }
 
@@ -416,8 +414,10 @@ int su2gpu_batch_create(su2gpu_batch **out, const su2gpu_batch_member *members, 
   for (int k = 0; k < 3 && e == hipSuccess; ++k) e = hipMalloc(&b->ar.U[k], b->ubytes);
   if (e == hipSuccess) e = hipMalloc(&b->ar.P, b->pelems * rb);
   if (e == hipSuccess) e = hipMalloc(&b->dlat, n * sizeof(su2k::BLat));
-  if (e == hipSuccess) e = hipMalloc(&b->dsums, n * 2 * NSUM * sizeof(double));
-  if (e == hipSuccess) e = hipHostMalloc(&b->hsums, n * 2 * NSUM * sizeof(double), hipHostMallocDefault);
+  // the reduction writes the sums itself to pinned coherent host memory
+  if (e == hipSuccess)
+    e = hipHostMalloc(&b->hsums, n * 2 * NSUM * sizeof(double), hipHostMallocMapped | hipHostMallocCoherent);
+  if (e == hipSuccess) e = hipHostGetDevicePointer((void **)&b->dsums, b->hsums, 0);
   if (e == hipSuccess) e = hipMalloc(&b->dtraj, sizeof(uint64_t));
   if (e == hipSuccess) e = hipHostMalloc(&b->htraj, sizeof(uint64_t), hipHostMallocDefault);
   int dev = 0;
@@ -459,7 +459,7 @@ int su2gpu_batch_destroy(su2gpu_batch *b) {
   for (int k = 0; k < 3; ++k)
     if (b->ar.U[k]) hipFree(b->ar.U[k]);
   for (void *p : {(void *)b->ar.P, (void *)b->dlat, (void *)b->dtiles, (void *)b->dltiles, (void *)b->partials,
-                  (void *)b->dsums, (void *)b->dtraj, (void *)b->staging})
+                  (void *)b->dtraj, (void *)b->staging})
     if (p) hipFree(p);
   for (void *p : {(void *)b->hsums, (void *)b->htraj, (void *)b->hstage})
     if (p) hipHostFree(p);

@@ -73,6 +73,9 @@ struct su2gpu_lattice {
   void *P = nullptr, *deriv = nullptr;
   double *partials = nullptr;
   int row_stride = 0;
+  // sums of the reduced rows, in pinned coherent host memory that the reduction
+  // writes itself (dsums: its device address): no copy between the reduction and
+  // the synchronisation (a copy took 4.3 us and a launch gap)
   double *dsums = nullptr, *hsums = nullptr;
   double *staging = nullptr;
   size_t staging_cap = 0;
@@ -352,8 +355,6 @@ int reduce_row(L *h, int r, int nb, su2k::RowList *defer = nullptr) {
   return defer ? SU2GPU_OK : reduce_rows(h, rl);
 }
 int fetch_sums(L *h) {
-  HC(hipMemcpyAsync(h->hsums, h->dsums, 2 * NROWS * sizeof(double), hipMemcpyDeviceToHost,
-                    h->stream));
   HC(hipStreamSynchronize(h->stream));
   return SU2GPU_OK;
 }
@@ -768,8 +769,9 @@ int su2gpu_create(su2gpu_lattice **out, int group, size_t Lx, size_t Ly, size_t 
   if (e == hipSuccess) e = hipMalloc(&h->U[2], h->U_bytes);
   if (e == hipSuccess) e = hipMalloc(&h->P, h->P_bytes);
   if (e == hipSuccess) e = hipMalloc(&h->partials, (size_t)NROWS * h->row_stride * sizeof(double));
-  if (e == hipSuccess) e = hipMalloc(&h->dsums, 2 * NROWS * sizeof(double));
-  if (e == hipSuccess) e = hipHostMalloc(&h->hsums, 2 * NROWS * sizeof(double), hipHostMallocDefault);
+  if (e == hipSuccess)
+    e = hipHostMalloc(&h->hsums, 2 * NROWS * sizeof(double), hipHostMallocMapped | hipHostMallocCoherent);
+  if (e == hipSuccess) e = hipHostGetDevicePointer((void **)&h->dsums, h->hsums, 0);
   if (e == hipSuccess) e = hipMemsetAsync(h->P, 0, h->P_bytes, h->stream);
   if (e != hipSuccess) {
     fail(SU2GPU_EHIP, "create: %s", hipGetErrorString(e));
@@ -807,7 +809,6 @@ int su2gpu_destroy(su2gpu_lattice *h) {
   if (h->P) hipFree(h->P);
   if (h->deriv) hipFree(h->deriv);
   if (h->partials) hipFree(h->partials);
-  if (h->dsums) hipFree(h->dsums);
   if (h->hsums) hipHostFree(h->hsums);
   if (h->staging) hipFree(h->staging);
   if (h->hstage) hipHostFree(h->hstage);
