@@ -25,6 +25,7 @@
 // not on the launch shape; it is not the reference's per-thread mt19937 stream.
 #include "su2_device.hpp"
 #include "su2_launch.hpp"
+#include "su2_md_plq.hpp"
 
 using namespace su2dev;
 
@@ -46,10 +47,52 @@ __device__ __forceinline__ double retr_mul_u1(double th, double kre, double kim)
   return c * kre - s * kim;
 }
 
+// sin(pi x) and cos(pi x): r = x - q / 2 exact, |r| <= 1/4, then the Taylor
+// series of both in (pi r)^2 <= 0.62 (remainders below 1e-18)
+__device__ __forceinline__ void sincospi_series(double x, double *sn, double *cs) {
+  const double q = rint(2.0 * x);
+  const double r = M_PI * fma(-0.5, q, x);
+  double c, s;
+  plq_series(r * r, c, s);
+  s *= r;
+  plq_quadrant((int)q, c, s);
+  *sn = s;
+  *cs = c;
+}
+
+// sqrt(x) for x in [2^-40, 2]: hardware estimate of 1/sqrt and two coupled
+// Newton steps (no scaling, no special values)
+__device__ __forceinline__ double sqrt_unit(double x) {
+  const double y = __builtin_amdgcn_rsq(x);
+  double g = x * y, h = 0.5 * y;
+  double e = fma(-h, g, 0.5);
+  g = fma(g, e, g);
+  h = fma(h, e, h);
+  return fma(fma(-g, g, x), h, g);
+}
+
+// v < exp(-dS): decided in FP32 where the two differ by more than 3e-5 of
+// their size (the FP32 exponential of an argument up to 100 is good to 1e-5;
+// beyond it is below every v > 2^-33), else, and for NaN, by the FP64 function
+__device__ __forceinline__ bool below_exp(double v, double dS) {
+  const float e = __expf(-(float)dS), w = (float)v;
+  if (w < e * (1.0f - 3e-5f)) return true;
+  if (w > e * (1.0f + 3e-5f)) return false;
+  return v < exp(-dS);
+}
+
+// What bounds it: at one hit the link gathers (every second site of a row: half
+// of each line a wave touches, 0.5 of the 0.68 ms of an FP64 32^4 sweep of 10
+// hits), beyond a few hits the vector units.  Against blocks dealt round the XCDs,
+// one direction at run time (a round trip per plane) and the library's sincospi,
+// sqrt, exp and division: FP64 32^4 10 hits 679 -> 520 us, 1 hit 517 -> 411 us, FP32
+// 570 -> 450 and 281 -> 218 us, U(1) 24^4 FP64 201 -> 153 us, three colours (15 21 7
+// 32) 168 -> 146 us.  With 4 waves per SIMD (128 registers); 3, 5 and 6: 520, 525,
+// 565 us.
 // list == nullptr: the sites of parity `parity` (every extent even);
 // otherwise the nlist sites list[0 .. nlist) of one colour class
-template <class G, int ND>
-__global__ __launch_bounds__(NTS) void k_sweep(typename G::link *__restrict__ U, Geo geo, int mu,
+template <class G, int ND, int mu>
+__global__ __launch_bounds__(NTS, 4) void k_sweep(typename G::link *__restrict__ U, Geo geo,
                                                int parity, const int *__restrict__ list,
                                                int nlist, uint64_t seed, uint64_t sweep,
                                                double delta, int n_hit, double beta_nc,
@@ -60,7 +103,16 @@ __global__ __launch_bounds__(NTS) void k_sweep(typename G::link *__restrict__ U,
   using acc = typename G::acc;
   __shared__ double lds[NTS / 64];
   const int V = geo.V;
-  const int j = blockIdx.x * NTS + threadIdx.x;
+  // each XCD walks one contiguous eighth of the sites; where the t slices divide
+  // into eighths and into blocks, with t fastest, so that a block's t neighbours
+  // were fetched by the blocks just before it into the same L2
+  int lb = xcd_block(blockIdx.x, gridDim.x);
+  if (!list && geo.L[0] % 8 == 0 && (V / 2 / geo.L[0]) % NTS == 0) {
+    const int nb3 = V / 2 / geo.L[0] / NTS, Tc = geo.L[0] / 8;
+    const int l = blockIdx.x >> 3, q = l / Tc;
+    lb = ((int)(blockIdx.x & 7) * Tc + l - q * Tc) * nb3 + q;
+  }
+  const int j = lb * NTS + threadIdx.x;
   double accepted = 0.0;
   if (list ? j < nlist : j < V / 2) {
     int s;
@@ -102,6 +154,15 @@ __global__ __launch_bounds__(NTS) void k_sweep(typename G::link *__restrict__ U,
     }
     const uint32_t lid = (uint32_t)s * (uint32_t)ND + (uint32_t)mu;
     link u = U[mu * V + s];
+    // ReTr(u K), kept from hit to hit
+    [[maybe_unused]] double retr;
+    [[maybe_unused]] quat<double> Kd;
+    if constexpr (G::NCOMP == 4) {
+      Kd = quat<double>{double(K.ar), double(K.ai), double(K.br), double(K.bi)};
+      retr = retr_mul(to_d(u), Kd);
+    } else {
+      retr = retr_mul_u1(double(u), double(K.re), double(K.im));
+    }
     for (int n = 0; n < n_hit; ++n) {
       uint32_t c[4] = {lid, (uint32_t)n, (uint32_t)(sweep & 0xffffffffu), (uint32_t)(sweep >> 32)};
       philox4x32_10(c, (uint32_t)seed, (uint32_t)(seed >> 32));
@@ -111,30 +172,32 @@ __global__ __launch_bounds__(NTS) void k_sweep(typename G::link *__restrict__ U,
         // alpha = 2 pi delta u0 and theta = 2 pi u2 through sincospi (no
         // argument reduction by pi)
         const double uu = -1.0 + 2.0 * u01_32(c[1]);
-        const double r = sqrt(1.0 - uu * uu);
+        const double r = sqrt_unit(1.0 - uu * uu);
         double sa, ca, st, ct;
-        sincospi(2.0 * delta * u01_32(c[0]), &sa, &ca);
-        sincospi(2.0 * u01_32(c[2]), &st, &ct);
+        sincospi_series(2.0 * delta * u01_32(c[0]), &sa, &ca);
+        sincospi_series(2.0 * u01_32(c[2]), &st, &ct);
         const quat<double> R{ca, sa * uu, sa * r * st, sa * r * ct};
-        const quat<double> ud{double(u.ar), double(u.ai), double(u.br), double(u.bi)};
-        const quat<double> Kd{double(K.ar), double(K.ai), double(K.br), double(K.bi)};
+        const quat<double> ud = to_d(u);
         const quat<double> uR = qmul(ud, R);
-        const double dS = beta_nc * (retr_mul(ud, Kd) - retr_mul(uR, Kd));
-        if (dS < 0.0 || v < exp(-dS)) {
-          // restoreSU (su2.hh:62-66) in FP64, one rounding to the storage precision
-          const double rn =
-              1.0 / sqrt(uR.ar * uR.ar + uR.ai * uR.ai + uR.br * uR.br + uR.bi * uR.bi);
+        const double dS = beta_nc * (retr - retr_mul(uR, Kd));
+        if (dS < 0.0 || below_exp(v, dS)) {
+          // restoreSU (su2.hh:62-66) in FP64, one rounding to the storage precision;
+          // 1/sqrt(1 + d) = 1 - d/2 + 3 d^2/8 - ... (5 d^3/16 < 4e-17 below 5e-6)
+          const double d = fma(uR.ar, uR.ar, fma(uR.ai, uR.ai, fma(uR.br, uR.br, fma(uR.bi, uR.bi, -1.0))));
+          const double rn = fabs(d) < 5e-6 ? fma(d, fma(0.375, d, -0.5), 1.0) : 1.0 / sqrt(1.0 + d);
           u = link{T(uR.ar * rn), T(uR.ai * rn), T(uR.br * rn), T(uR.bi * rn)};
+          retr = retr_mul(to_d(u), Kd);
           accepted += 1.0;
         }
       } else {
         // random_element (random_element.hh:27-34): phase in [-pi delta, pi delta)
         const double th = -M_PI * delta + (2.0 * M_PI * delta) * u01_32(c[0]);
         const double ud = double(u), un = ud + th;
-        const double dS = beta_nc * (retr_mul_u1(ud, double(K.re), double(K.im)) -
-                                     retr_mul_u1(un, double(K.re), double(K.im)));
-        if (dS < 0.0 || v < exp(-dS)) {
+        const double rn = retr_mul_u1(un, double(K.re), double(K.im));
+        const double dS = beta_nc * (retr - rn);
+        if (dS < 0.0 || below_exp(v, dS)) {
           u = T(un);
+          retr = sizeof(T) == 8 ? rn : retr_mul_u1(double(u), double(K.re), double(K.im));
           accepted += 1.0;
         }
       }
@@ -142,32 +205,26 @@ __global__ __launch_bounds__(NTS) void k_sweep(typename G::link *__restrict__ U,
     U[mu * V + s] = u;
   }
   const double r = block_sum<NTS>(accepted, lds);
-  if (threadIdx.x == 0) partials[blockIdx.x] = r;
+  if (threadIdx.x == 0) partials[lb] = r;
 }
 
 int sweep_blocks(const Geo &g, int nlist) { return ((nlist >= 0 ? nlist : g.V / 2) + NTS - 1) / NTS; }
 
-template <class G>
-static void sweep_g(void *U, const Geo &g, int mu, int parity, const int *list, int nlist,
-                    uint64_t seed, uint64_t sweep, double delta, int n_hit, double beta_nc,
-                    double w_t, double w_s, int aniso, double *partials, hipStream_t st) {
+template <class G, int ND>
+static void sweep_nd(void *U, const Geo &g, int mu, int parity, const int *list, int nlist,
+                     uint64_t seed, uint64_t sweep, double delta, int n_hit, double beta_nc,
+                     double w_t, double w_s, int aniso, double *partials, hipStream_t st) {
   using link = typename G::link;
   const dim3 grid(sweep_blocks(g, list ? nlist : -1));
   if (grid.x == 0) return;
-  switch (g.nd) {
-    case 2:
-      hipLaunchKernelGGL((k_sweep<G, 2>), grid, dim3(NTS), 0, st, (link *)U, g, mu, parity, list,
-                         nlist, seed, sweep, delta, n_hit, beta_nc, w_t, w_s, aniso, partials);
-      break;
-    case 3:
-      hipLaunchKernelGGL((k_sweep<G, 3>), grid, dim3(NTS), 0, st, (link *)U, g, mu, parity, list,
-                         nlist, seed, sweep, delta, n_hit, beta_nc, w_t, w_s, aniso, partials);
-      break;
-    default:
-      hipLaunchKernelGGL((k_sweep<G, 4>), grid, dim3(NTS), 0, st, (link *)U, g, mu, parity, list,
-                         nlist, seed, sweep, delta, n_hit, beta_nc, w_t, w_s, aniso, partials);
-      break;
-  }
+#define SU2_SWEEP(M)                                                                          \
+  hipLaunchKernelGGL((k_sweep<G, ND, M>), grid, dim3(NTS), 0, st, (link *)U, g, parity, list, \
+                     nlist, seed, sweep, delta, n_hit, beta_nc, w_t, w_s, aniso, partials)
+  if (mu == 0) SU2_SWEEP(0);
+  else if (mu == 1) SU2_SWEEP(1);
+  else if (ND > 2 && mu == 2) SU2_SWEEP((ND > 2 ? 2 : 0));
+  else SU2_SWEEP((ND > 3 ? 3 : 0));
+#undef SU2_SWEEP
 }
 
 void launch_sweep(int group, int prec, void *U, const Geo &g, int mu, int parity, const int *list,
@@ -175,13 +232,20 @@ void launch_sweep(int group, int prec, void *U, const Geo &g, int mu, int parity
                   double beta_nc, double w_t, double w_s, int aniso, double *partials,
                   hipStream_t st) {
 #define SWEEP_ARGS U, g, mu, parity, list, nlist, seed, sweep, delta, n_hit, beta_nc, w_t, w_s, aniso, partials, st
+#define SWEEP_G(G)                               \
+  do {                                           \
+    if (g.nd == 2) sweep_nd<G, 2>(SWEEP_ARGS);   \
+    else if (g.nd == 3) sweep_nd<G, 3>(SWEEP_ARGS); \
+    else sweep_nd<G, 4>(SWEEP_ARGS);             \
+  } while (0)
   if (group == 1) {
-    if (prec == 0) sweep_g<GSU2<double>>(SWEEP_ARGS);
-    else sweep_g<GSU2<float>>(SWEEP_ARGS);
+    if (prec == 0) SWEEP_G(GSU2<double>);
+    else SWEEP_G(GSU2<float>);
   } else {
-    if (prec == 0) sweep_g<GU1<double>>(SWEEP_ARGS);
-    else sweep_g<GU1<float>>(SWEEP_ARGS);
+    if (prec == 0) SWEEP_G(GU1<double>);
+    else SWEEP_G(GU1<float>);
   }
+#undef SWEEP_G
 #undef SWEEP_ARGS
 }
 
