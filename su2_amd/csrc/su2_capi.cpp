@@ -763,6 +763,7 @@ int su2gpu_create(su2gpu_lattice **out, int group, size_t Lx, size_t Ly, size_t 
   hipError_t e = hipGetDevice(&h->device);
   if (e == hipSuccess) e = hipStreamCreateWithFlags(&h->stream, hipStreamNonBlocking);
   h->row_stride = std::max({su2k::fused_blocks(h->geo), su2k::plq_partials(group, precision, h->geo),
+                            su2k::clover_partials(group, precision, h->geo),
                             su2k::sumsq_blocks((long)h->nlinks * h->nm)});
   if (e == hipSuccess) e = hipMalloc(&h->U[0], h->U_bytes);
   if (e == hipSuccess) e = hipMalloc(&h->U[1], h->U_bytes);
@@ -1234,23 +1235,16 @@ int su2gpu_md_update(su2gpu_lattice *h, uint64_t seed, int integrator, size_t ns
   return su2gpu_md_finish(h, accept);
 }
 
-int su2gpu_energy_density(su2gpu_lattice *h, int clover, int ss, double *E, double *Q) {
-  CK(check(h));
-  if (!E || !Q) return fail(SU2GPU_EINVAL, "null pointer");
-  const int nbf = su2k::site_blocks(h->geo);
-  {
-    Prof pr(h, "energy_density");
-    su2k::launch_energy_density(h->group, h->prec, h->U[h->cur], h->geo, clover ? 1 : 0,
-                                ss ? 1 : 0, row(h, 20), h->row_stride, h->stream);
-  }
-  CK(last_launch("energy_density"));
-  su2k::RowList rl;
-  CK(reduce_row(h, 20, nbf, &rl));
-  CK(reduce_row(h, 21, nbf, &rl));
-  CK(reduce_rows(h, rl));
-  CK(fetch_sums(h));
-  long double e = sum_of(h, 20), q = sum_of(h, 21);
-  // flat-energy_density.hh:152-163
+namespace {
+// plaquette sums (gauge_energy of all and of the spatial planes) and clover energy
+// density and charge, of all and of the spatial planes
+struct Observables {
+  double plaq, plaq_ss, E, Q, E_ss, Q_ss;
+};
+enum : int { OBS_PLAQ = 1, OBS_PLAQ_SS = 2, OBS_E = 4, OBS_E_SS = 8 };
+
+// flat-energy_density.hh:152-163
+void density(const L *h, int clover, long double e, long double q, double *E, double *Q) {
   double res = -(double)e / (double)h->V;
   if (clover) res /= 16.;
   double qq = -4. * (double)q / (32.0 * M_PI * M_PI);
@@ -1258,6 +1252,79 @@ int su2gpu_energy_density(su2gpu_lattice *h, int clover, int ss, double *E, doub
   if (h->nd == 3) qq = 0.0;
   *E = res;
   *Q = qq;
+}
+
+// the wanted observables of the handle's links with one reduction and one
+// synchronisation: the fused pass (launch_clover) where it applies and a clover
+// observable is wanted, else the separate kernels
+int observables(L *h, int want, Observables *o) {
+  constexpr int R0 = 20;
+  su2k::RowList rl;
+  int nb = 0;
+  if (want & (OBS_E | OBS_E_SS)) {
+    Prof pr(h, "energy_density");
+    nb = su2k::launch_clover(h->group, h->prec, h->U[h->cur], h->geo, row(h, R0), h->row_stride,
+                             h->stream);
+  }
+  CK(last_launch("energy_density"));
+  if (nb > 0) {
+    for (int r = 0; r < 5; ++r) CK(reduce_row(h, R0 + r, nb, &rl));
+    CK(reduce_rows(h, rl));
+    CK(fetch_sums(h));
+    const long double ps = sum_of(h, R0 + 1), es = sum_of(h, R0 + 3);
+    o->plaq = (double)(sum_of(h, R0) + ps);
+    o->plaq_ss = (double)ps;
+    density(h, 1, sum_of(h, R0 + 2) + es, sum_of(h, R0 + 4), &o->E, &o->Q);
+    density(h, 1, es, 0.0L, &o->E_ss, &o->Q_ss);
+    return SU2GPU_OK;
+  }
+  if (want & OBS_PLAQ) CK(plaq_launch(h, h->cur, -1, 1.0, 1.0, 0, 0, R0 + 4, &rl));
+  if (want & OBS_PLAQ_SS) CK(plaq_launch(h, h->cur, -1, 1.0, 1.0, 1, 0, R0 + 5, &rl));
+  const int nbf = su2k::site_blocks(h->geo);
+  for (int ss = 0; ss < 2; ++ss) {
+    if (!(want & (ss ? OBS_E_SS : OBS_E))) continue;
+    {
+      Prof pr(h, "energy_density");
+      su2k::launch_energy_density(h->group, h->prec, h->U[h->cur], h->geo, 1, ss,
+                                  row(h, R0 + 2 * ss), h->row_stride, h->stream);
+    }
+    CK(last_launch("energy_density"));
+    CK(reduce_row(h, R0 + 2 * ss, nbf, &rl));
+    CK(reduce_row(h, R0 + 2 * ss + 1, nbf, &rl));
+  }
+  CK(reduce_rows(h, rl));
+  CK(fetch_sums(h));
+  if (want & OBS_PLAQ) o->plaq = (double)sum_of(h, R0 + 4);
+  if (want & OBS_PLAQ_SS) o->plaq_ss = (double)sum_of(h, R0 + 5);
+  if (want & OBS_E) density(h, 1, sum_of(h, R0), sum_of(h, R0 + 1), &o->E, &o->Q);
+  if (want & OBS_E_SS) density(h, 1, sum_of(h, R0 + 2), sum_of(h, R0 + 3), &o->E_ss, &o->Q_ss);
+  return SU2GPU_OK;
+}
+}  // namespace
+
+int su2gpu_energy_density(su2gpu_lattice *h, int clover, int ss, double *E, double *Q) {
+  CK(check(h));
+  if (!E || !Q) return fail(SU2GPU_EINVAL, "null pointer");
+  if (clover) {
+    Observables o{};
+    CK(observables(h, ss ? OBS_E_SS : OBS_E, &o));
+    *E = ss ? o.E_ss : o.E;
+    *Q = ss ? o.Q_ss : o.Q;
+    return SU2GPU_OK;
+  }
+  const int nbf = su2k::site_blocks(h->geo);
+  {
+    Prof pr(h, "energy_density");
+    su2k::launch_energy_density(h->group, h->prec, h->U[h->cur], h->geo, 0, ss ? 1 : 0, row(h, 20),
+                                h->row_stride, h->stream);
+  }
+  CK(last_launch("energy_density"));
+  su2k::RowList rl;
+  CK(reduce_row(h, 20, nbf, &rl));
+  CK(reduce_row(h, 21, nbf, &rl));
+  CK(reduce_rows(h, rl));
+  CK(fetch_sums(h));
+  density(h, 0, sum_of(h, 20), sum_of(h, 21), E, Q);
   return SU2GPU_OK;
 }
 
@@ -1402,16 +1469,13 @@ int su2gpu_gradient_flow(su2gpu_lattice *h, double tmax, double eps, double tsta
   for (int i = 0; i < 3; ++i) t[i] = tstart;
   int rc = SU2GPU_OK;
   auto measure = [&](int k, bool withQ) -> int {
-    double g, gss, e, q, ess, qss;
-    CK(su2gpu_gauge_energy(h, 0, &g));
-    CK(su2gpu_gauge_energy(h, 1, &gss));
-    CK(su2gpu_energy_density(h, 1, 0, &e, &q));
-    CK(su2gpu_energy_density(h, 1, 1, &ess, &qss));
-    P[k] = g / den;
-    Pss[k] = gss / den;
-    E[k] = e;
-    Ess[k] = ess;
-    if (withQ) Q[k] = q;
+    Observables o{};
+    CK(observables(h, OBS_PLAQ | OBS_PLAQ_SS | OBS_E | OBS_E_SS, &o));
+    P[k] = o.plaq / den;
+    Pss[k] = o.plaq_ss / den;
+    E[k] = o.E;
+    Ess[k] = o.E_ss;
+    if (withQ) Q[k] = o.Q;
     return SU2GPU_OK;
   };
   h->cur = vt;

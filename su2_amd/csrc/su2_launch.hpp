@@ -103,6 +103,14 @@ void launch_reduce(const double *partials, size_t row_stride, const RowList &rl,
                    hipStream_t st);
 void launch_energy_density(int group, int prec, const void *U, const Geo &g, int clover,
                            int mu_start, double *partials, int pstride, hipStream_t st);
+// SU(2), d = 4: the plaquette and clover sums of one configuration in one pass
+// (su2_clover.hip), rows of partials pstride apart: 0 / 1 the temporal / spatial
+// plaquettes, 2 / 3 the temporal / spatial planes' ReTr(G G), 4 the charge sum of
+// k_energy_density.  Returns the block partials per row, 0 where it does not
+// apply (nothing launched); clover_partials: that number.
+int launch_clover(int group, int prec, const void *U, const Geo &g, double *partials, int pstride,
+                  hipStream_t st);
+int clover_partials(int group, int prec, const Geo &g);
 void launch_links_from_aos(int group, int prec, const double *src, int stride, int offset,
                            void *dst, int V, int nd, hipStream_t st);
 void launch_links_to_aos(int group, int prec, const void *src, double *dst, int stride,

@@ -128,8 +128,8 @@ inline uint32_t plq_threads(const PlqGeo &g) {
 
 // The rows of a block for extents L (t, x, y, z; nd = 3, 4); false where the
 // step does not apply.  rpb: the rows that waste the fewest lanes of at most
-// 256 threads, fewer edge rows breaking ties.
-inline bool make_plq_rows(const int L[4], int nd, int V, PlqGeo &g) {
+// `threads`, fewer edge rows breaking ties.
+inline bool make_plq_rows(const int L[4], int nd, int V, PlqGeo &g, int threads = PLQ_NT) {
   if (nd < 3 || nd > 4) return false;
   for (int k = 0; k < 4; ++k) g.L[k] = L[k];
   g.nd = nd;
@@ -146,7 +146,7 @@ inline bool make_plq_rows(const int L[4], int nd, int V, PlqGeo &g) {
   if ((uint64_t)V * 32u >= two32) return false;  // 32-bit byte offsets in a plane
   double best = 0.0;
   g.rpb = 0;
-  for (int r = 1; r <= g.nrows && r * Lf <= PLQ_NT; ++r) {
+  for (int r = 1; r <= g.nrows && r * Lf <= threads; ++r) {
     const int nyb = (g.nrows + r - 1) / r, nt = (r * Lf + 63) / 64 * 64;
     // useful rows per lane, less the edge rows' terms (a fifth of a row each,
     // none where the block holds every row)
