@@ -124,6 +124,7 @@ struct su2gpu_lattice {
     void *Zs[2] = {nullptr, nullptr};   // Z after stages 0 and 1
     void *lamW = nullptr, *lamZ = nullptr, *Gam = nullptr;
     void *R = nullptr;                  // scratch of the adjoint's plaquette pass
+    void *lz[2] = {nullptr, nullptr};   // lambda_Z records of the one-pass stage, in turn
     std::vector<void *> stU, stZ;       // stage states of a segment: W1, W2 and Z0', Z1', Z2' per step
     bool kept_last = false;             // the forward left the last segment's states in seg/stU/stZ
   } flow;
@@ -802,7 +803,8 @@ int su2gpu_destroy(su2gpu_lattice *h) {
     for (void *p : f.seg) hipFree(p);
     for (void *p : f.stU) hipFree(p);
     for (void *p : f.stZ) hipFree(p);
-    for (void *p : {f.W[0], f.W[1], f.Z, f.W1, f.W2, f.Zs[0], f.Zs[1], f.lamW, f.lamZ, f.Gam, f.R})
+    for (void *p : {f.W[0], f.W[1], f.Z, f.W1, f.W2, f.Zs[0], f.Zs[1], f.lamW, f.lamZ, f.Gam, f.R, f.lz[0],
+                    f.lz[1]})
       if (p) hipFree(p);
   }
   for (int i = 0; i < NBUF; ++i)
@@ -1570,6 +1572,9 @@ int rk_step(L *h, const void *Win, void *Wout, void *tmp, void *Z, double eps) {
 }  // namespace
 
 namespace {
+// one lambda_Z field of the one-pass stage: four reals per link
+size_t lz_bytes(const L *h) { return (size_t)h->nlinks * 4 * h->real_bytes; }
+
 // buffers for the stage states of one segment (seg: W_k, stU: W1 W2, stZ: the
 // three Z' per step), kept when they fit in half of the free device memory
 // and SU2GPU_FLOW_RECOMPUTE is not set; false: recompute per step instead
@@ -1585,14 +1590,20 @@ int flow_keep_buffers(L *h, bool *keep) {
   if (*keep && f.stU.size() < 2 * f.ckpt) {
     size_t fr = 0, tot = 0;
     HC(hipMemGetInfo(&fr, &tot));
-    // the backward pass's own fields (W2, Zs[2], lamW, lamZ, the 36 V scratch
-    // R and the 18 V clover cotangent Gam) count against the same free memory
+    // the backward pass's own fields (W2, Zs[2], lamW, lamZ and the 36 V scratch R
+    // or the two lambda_Z records, and the 18 V clover cotangent Gam) count against the same free memory
     // when it has not allocated them yet
     size_t bwd = 0;
     if (!f.W2) bwd += h->U_bytes;
-    for (void *p : {f.Zs[0], f.Zs[1], f.lamW, f.lamZ})
+    for (void *p : {f.Zs[0], f.Zs[1], f.lamW})
       if (!p) bwd += h->P_bytes;
-    if (!f.R) bwd += (size_t)h->V * 36 * h->real_bytes;
+    if (su2k::flow_fused_ok(h->prec, h->geo)) {
+      for (void *p : f.lz)
+        if (!p) bwd += lz_bytes(h);
+    } else {
+      if (!f.lamZ) bwd += h->P_bytes;
+      if (!f.R) bwd += (size_t)h->V * 36 * h->real_bytes;
+    }
     if (!f.Gam) bwd += (size_t)h->V * 18 * h->real_bytes;
     const size_t need = (2 * f.ckpt - f.stU.size()) * h->U_bytes +
                         (3 * f.ckpt - f.stZ.size()) * h->P_bytes + bwd;
@@ -1712,8 +1723,13 @@ int su2gpu_flow_backward(su2gpu_lattice *h, double *grad) {
   CK(flow_alloc(h, &f.Zs[0], h->P_bytes));
   CK(flow_alloc(h, &f.Zs[1], h->P_bytes));
   CK(flow_alloc(h, &f.lamW, h->P_bytes));
-  CK(flow_alloc(h, &f.lamZ, h->P_bytes));
-  CK(flow_alloc(h, &f.R, (size_t)h->V * 36 * h->real_bytes));
+  const bool fused_stage = su2k::flow_fused_ok(h->prec, h->geo);
+  if (fused_stage) {
+    for (auto &p : f.lz) CK(flow_alloc(h, &p, lz_bytes(h)));
+  } else {
+    CK(flow_alloc(h, &f.lamZ, h->P_bytes));
+    CK(flow_alloc(h, &f.R, (size_t)h->V * 36 * h->real_bytes));
+  }
   const double w_t = h->aniso ? 1.0 / h->xi : 1.0, w_s = h->aniso ? h->xi : 1.0;
   // cotangent of W(t)
   const double t = f.eps * (double)f.nsteps;
@@ -1744,8 +1760,22 @@ int su2gpu_flow_backward(su2gpu_lattice *h, double *grad) {
   // The gather of a stage's Hessian-vector product (the b/c role terms in R)
   // runs fused with the pointwise adjoint of the stage before it; the stage
   // recomputation in between touches neither R nor lamW / lamZ.
+  // In the one-pass form a stage's product waits for the Z' of the stage before it
+  // (or, at the end of a segment, whose links the next one's recomputation
+  // overwrites, runs alone).
   bool pending = false;
   double pending_b = 0.0;
+  const void *pending_W = nullptr;
+  int lzc = 0;  // the lambda_Z record field last written
+  auto fused_product = [&](const void *Z, double cz, int zero_lamZ) -> int {
+    {
+      Prof pr(h, "flow_vjp");
+      su2k::launch_flow_fused(pending_W, f.lz[lzc], f.lz[1 - lzc], f.lamW, Z, h->geo, pending_b, w_t,
+                              w_s, cz, zero_lamZ, h->stream);
+    }
+    if (Z) lzc = 1 - lzc;
+    return last_launch("flow_fused");
+  };
   const size_t nseg = f.ckpts.size();
   for (size_t sg = nseg; sg-- > 0;) {
     const size_t k0 = sg * f.ckpt, k1 = std::min(f.nsteps, k0 + f.ckpt);
@@ -1784,6 +1814,19 @@ int su2gpu_flow_backward(su2gpu_lattice *h, double *grad) {
         CK(rk_stage(h, f.W2, nullptr, f.Zs[1], b[2], c[2], false, f.Z));
       }
       for (int st = 2; st >= 0; --st) {
+        if (fused_stage) {
+          if (pending) {
+            CK(fused_product(Zst[st], c[st], st == 2 ? 1 : 0));
+          } else {
+            Prof pr(h, "flow_stage_adj");
+            su2k::launch_flow_first_adj(Zst[st], f.lamW, f.lz[lzc], h->geo, c[st], h->stream);
+          }
+          CK(last_launch("flow_stage_adj"));
+          pending = true;
+          pending_b = b[st];
+          pending_W = Wst[st];
+          continue;
+        }
         {
           Prof pr(h, "flow_stage_adj");
           if (pending)
@@ -1803,6 +1846,10 @@ int su2gpu_flow_backward(su2gpu_lattice *h, double *grad) {
         pending = true;
         pending_b = b[st];
       }
+    }
+    if (fused_stage && pending) {
+      CK(fused_product(nullptr, 0.0, 0));
+      pending = false;
     }
   }
   if (pending) {

@@ -147,6 +147,16 @@ void launch_flow_gather(int prec, const void *R, void *lamW, const Geo &g, doubl
 void launch_flow_gather_stage_adj(int prec, const void *R, void *lamW, void *lamZ, const void *Zs,
                                   const Geo &g, double b, double c, int zero_lamZ,
                                   hipStream_t st);
+// the same stage in one pass (su2_flow_plq.hip; SU(2) d = 4, FP32): the product
+// of one stage and, where Zs is given, the pointwise adjoint of the stage before it.
+// lambda_Z in records of 4 reals per link, read from lzi and written to lzo;
+// launch_flow_first_adj: the pointwise adjoint alone, lambda_Z from zero to lzo
+bool flow_fused_ok(int prec, const Geo &g);
+void launch_flow_first_adj(const void *Zs, void *lamW, void *lzo, const Geo &g, double c,
+                           hipStream_t st);
+void launch_flow_fused(const void *U, const void *lzi, void *lzo, void *lamW, const void *Zs,
+                       const Geo &g, double b, double w_t, double w_s, double c, int zero_lamZ,
+                       hipStream_t st);
 void launch_clover_grad(int prec, const void *U, void *Gam, void *lamW, const Geo &g,
                         double scale, hipStream_t st);
 
