@@ -16,7 +16,7 @@ LIB = os.path.join(HERE, "libsu2mi355x.so")
 OBJDIR = os.path.join(HERE, "_build")
 
 SOURCES = ["su2_kernels.hip", "su2_flow.hip", "su2_batch.hip", "su2_sweep.hip", "su2_plq.hip", "su2_clover.hip",
-           "su2_flow_plq.hip",
+           "su2_flow_plq.hip", "su2_batch_plq.hip",
            "su2_capi.cpp",
            "su2_batch.cpp", "su2_noalloc.hip"]
 HEADERS = ["su2_device.hpp", "su2_launch.hpp"]
@@ -31,9 +31,9 @@ HIPCC_FLAGS = [
 # machine LICM moves FP64 literals out of the loops into vector registers, which
 # these kernels have none to spare of (the shared-plaquette step: 87 against 10
 # spilled registers; the sweep: 72 against 58 in use)
-EXTRA_FLAGS = {s: ["-mllvm", "-disable-machine-licm"] 
-               for s in ("su2_plq.hip", "su2_clover.hip", "su2_flow_plq.hip",
-                                                                "su2_sweep.hip")}
+EXTRA_FLAGS = {s: ["-mllvm", "-disable-machine-licm"]
+               for s in ("su2_plq.hip", "su2_clover.hip", "su2_flow_plq.hip", "su2_batch_plq.hip",
+                         "su2_sweep.hip")}
 
 
 def hipcc() -> str:

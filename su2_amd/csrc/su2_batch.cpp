@@ -69,6 +69,18 @@ struct su2gpu_batch {
       maxpairs = 0;
   // active[3 t + k]: leading link tiles of part k whose lattices still run at tick t
   std::vector<int> active;
+  // the d = 4 part on the shared-plaquette tiles: plans of falling size, tick t
+  // runs the first `count` tiles of plan ptick[t] (-1: its link tiles)
+  struct PlqPlan {
+    void *geos = nullptr;
+    int2 *tiles = nullptr;
+    unsigned threads = 0, lds = 0;
+  };
+  std::vector<PlqPlan> plans;
+  struct PlqTick {
+    int plan = -1, count = 0;
+  };
+  std::vector<PlqTick> ptick;
   double *partials = nullptr, *dsums = nullptr, *hsums = nullptr;
   uint64_t *dtraj = nullptr, *htraj = nullptr;
   double *staging = nullptr, *hstage = nullptr;
@@ -93,6 +105,51 @@ namespace {
 using B = su2gpu_batch;
 
 int npairs_of(int kind, size_t n) { return kind == SU2GPU_OMF2 ? (int)(2 * n) : (int)n; }
+
+void free_plans(B *b) {
+  for (auto &q : b->plans) {
+    if (q.geos) (void)hipFree(q.geos);
+    if (q.tiles) (void)hipFree(q.tiles);
+  }
+  b->plans.clear();
+}
+
+// The shared-plaquette tiles of the d = 4 part, from how many running sites on its
+// ticks take them.  The slices of a chunk are chosen for the lattices still
+// running: a new plan whenever their sites fell below three quarters of the last
+// plan's.
+int build_plq(B *b, const std::vector<size_t> &order) {
+  free_plans(b);
+  b->ptick.assign(b->maxpairs + 1, B::PlqTick{});
+  std::vector<size_t> part;
+  for (size_t l : order)
+    if (b->lat[l].spec == 4) part.push_back(l);
+  double planned = 0.0;
+  std::vector<int> end;
+  for (int t = 0; t <= b->maxpairs; ++t) {
+    while (!part.empty() && b->lat[part.back()].npairs < t) part.pop_back();
+    double run = 0.0;
+    for (size_t l : part) run += b->lat[l].geo.V;
+    if (run < su2k::batch_plq_sites(b->prec)) break;
+    if (b->plans.empty() || run < 0.75 * planned) {
+      su2k::BatchPlqPlan p;
+      if (!su2k::plan_batch_plq(b->prec, b->ncu, b->lat, part, p)) break;
+      b->plans.emplace_back();
+      auto &q = b->plans.back();
+      q.threads = p.threads;
+      q.lds = p.lds;
+      BH(hipMalloc(&q.tiles, p.tiles.size() * sizeof(int2)));
+      BH(hipMemcpy(q.tiles, p.tiles.data(), p.tiles.size() * sizeof(int2), hipMemcpyHostToDevice));
+      BH(hipMalloc(&q.geos, p.geos.size()));
+      BH(hipMemcpy(q.geos, p.geos.data(), p.geos.size(), hipMemcpyHostToDevice));
+      planned = run;
+      end.assign(b->lat.size(), 0);
+      for (size_t i = 0; i < p.tiles.size(); ++i) end[p.tiles[i].x] = (int)i + 1;
+    }
+    b->ptick[t] = {(int)b->plans.size() - 1, end[part.back()]};
+  }
+  return SU2GPU_OK;
+}
 
 // site tiles (tile size = block) and link tiles (one per site tile and mu, mu
 // fastest, site start packed as 4*s + mu); lattices contiguous
@@ -135,6 +192,7 @@ int build_tiles(B *b) {
     }
     if (pass == 4) b->nspec4 = (int)ltiles.size() - before;
     if (pass == 3) b->nspec3 = (int)ltiles.size() - before;
+    if (pass == 4) BK(build_plq(b, order));
   }
   b->ntiles = (int)tiles.size();
   b->nltiles = (int)ltiles.size();
@@ -219,6 +277,18 @@ int enqueue(B *b, bool devmom, Rec *rec = nullptr) {
                           b->partials, b->grid_site, b->block, b->stream);
   fin();
   const int flags = (b->prec == 1) ? (su2k::F_COMPENSATED | su2k::F_RESTORE) : 0;
+  auto tick = [&](int t, int part, hipStream_t st) {
+    const auto pt = part == 0 ? b->ptick[t] : B::PlqTick{};
+    if (pt.plan >= 0) {
+      const auto &q = b->plans[pt.plan];
+      su2k::launch_batch_plq(b->prec, b->dlat, q.geos, q.tiles, pt.count, b->nltiles, b->ar, t,
+                             flags, b->partials, q.threads, q.lds, st);
+    } else {
+      su2k::launch_batch_tick(b->prec, b->dlat, b->dltiles, b->nltiles, b->nspec4, b->nspec3,
+                              b->ar, t, flags, b->partials, b->grid, b->block, st, part,
+                              &b->active[3 * t]);
+    }
+  };
   if (!rec && b->concurrent) {
     // three independent tick chains: d = 4 on `stream`, d = 3 and the rest on
     // the part streams, joined before the final sums
@@ -226,29 +296,18 @@ int enqueue(B *b, bool devmom, Rec *rec = nullptr) {
     for (int k = 0; k < 2; ++k) BH(hipStreamWaitEvent(b->pstream[k], b->ev_fork, 0));
     for (int t = 0; t <= b->maxpairs; ++t)
       for (int part = 0; part < 3; ++part)
-        su2k::launch_batch_tick(b->prec, b->dlat, b->dltiles, b->nltiles, b->nspec4, b->nspec3,
-                                b->ar, t, flags, b->partials, b->grid, b->block,
-                                part == 0 ? b->stream : b->pstream[part - 1], part,
-                                &b->active[3 * t]);
+        tick(t, part, part == 0 ? b->stream : b->pstream[part - 1]);
     for (int k = 0; k < 2; ++k) {
       BH(hipEventRecord(b->ev_join[k], b->pstream[k]));
       BH(hipStreamWaitEvent(b->stream, b->ev_join[k], 0));
     }
-  }
-  for (int t = 0; t <= b->maxpairs && (rec || !b->concurrent); ++t) {
-    if (!rec) {
-      su2k::launch_batch_tick(b->prec, b->dlat, b->dltiles, b->nltiles, b->nspec4, b->nspec3,
-                              b->ar, t, flags, b->partials, b->grid, b->block, b->stream, -1,
-                              &b->active[3 * t]);
-      continue;
-    }
-    for (int part = 0; part < 3; ++part) {
-      beg(RK_TICK4 + part);
-      su2k::launch_batch_tick(b->prec, b->dlat, b->dltiles, b->nltiles, b->nspec4, b->nspec3,
-                              b->ar, t, flags, b->partials, b->grid, b->block, b->stream, part,
-                              &b->active[3 * t]);
-      fin();
-    }
+  } else {
+    for (int t = 0; t <= b->maxpairs; ++t)
+      for (int part = 0; part < 3; ++part) {
+        beg(RK_TICK4 + part);
+        tick(t, part, b->stream);
+        fin();
+      }
   }
   if (b->prec == 0) {
     beg(RK_RESTORE);
@@ -478,6 +537,7 @@ int su2gpu_batch_destroy(su2gpu_batch *b) {
   if (b->graph) hipGraphDestroy(b->graph);
   for (int k = 0; k < 3; ++k)
     if (b->ar.U[k]) hipFree(b->ar.U[k]);
+  free_plans(b);
   for (void *p : {(void *)b->ar.P, (void *)b->dlat, (void *)b->dtiles, (void *)b->dltiles, (void *)b->partials,
                   (void *)b->dtraj, (void *)b->staging})
     if (p) hipFree(p);

@@ -5,8 +5,9 @@
 // cut into tiles of `tile` sites; one MD tick (one "P then U" pair of every
 // lattice's integrator, or its final momentum step) is three launches of a
 // grid-stride kernel: over the tiles of the SU(2) lattices in d = 4, in d = 3
-// (the specialised step body of su2_md_fast.hpp), and over the rest, whatever the
-// lattice's group and dimension: a tile selects its (group, d) code path
+// (the specialised step body of su2_md_fast.hpp; in d = 4 the shared-plaquette
+// step of su2_batch_plq.hip while enough sites run), and over the rest, whatever
+// the lattice's group and dimension: a tile selects its (group, d) code path
 // uniformly for the block.
 // Lattice l's k-th link update reads arena r(k) and writes w(k) with
 //   r(0) = a0, r(k>0) = (k odd ? a1 : a2), w(k) = (k even ? a1 : a2),
@@ -20,19 +21,6 @@
 using namespace su2dev;
 
 namespace su2k {
-
-// integrator pair k of lattice l: (P coefficient, U coefficient) in units of dtau
-__device__ __forceinline__ void pair_coef(int kind, int k, double &cp, double &cu) {
-  if (kind == 6) {  // omf2 (integrator.hh:83-115): P(l) [U(1/2) P(1-2l) U(1/2) P(2l)]... P(l)
-    const double lam = 0.1938;
-    cp = (k == 0) ? lam : ((k & 1) ? 1. - 2. * lam : 2. * lam);
-    cu = 0.5;
-  } else {  // leapfrog (integrator.hh:26-50): P(1/2) U(1) [P(1) U(1)]... P(1/2)
-    cp = (k == 0) ? 0.5 : 1.0;
-    cu = 1.0;
-  }
-}
-__device__ __forceinline__ double final_coef(int kind) { return kind == 6 ? 0.1938 : 0.5; }
 
 // SU(2) in d = 3, 4: the specialised step body (mu selects one of ND compiled
 // bodies; it is uniform over the tile), neighbour offsets from the lattice's
@@ -114,27 +102,11 @@ __global__ __launch_bounds__(256) void k_batch_tick(const BLat *__restrict__ lat
     const BLat &L = lats[tl.x];
     if (tick > L.npairs) continue;  // lattice finished (uniform over the block)
     const int s = (tl.y >> 2) + threadIdx.x, mu = tl.y & 3;
-    const int a0 = L.cur, a1 = (L.cur + 1) % 3, a2 = (L.cur + 2) % 3;
-    FusedCoef c{};
-    c.coef = L.coef;
-    c.w_t = 1.0;
-    c.w_s = 1.0;
-    c.flags = flags;
     double k0 = 0.0, act = 0.0, k1 = 0.0;
     const bool final_p = (tick == L.npairs);
+    FusedCoef c{};
     int rd, wr;
-    if (!final_p) {
-      double cp, cu;
-      pair_coef(L.kind, tick, cp, cu);
-      c.ep = cp * L.dtau;
-      c.eu = cu * L.dtau;
-      rd = (tick == 0) ? a0 : ((tick & 1) ? a1 : a2);
-      wr = (tick & 1) ? a2 : a1;
-    } else {
-      c.ep = final_coef(L.kind) * L.dtau;
-      rd = L.npairs == 0 ? a0 : (((L.npairs - 1) & 1) ? a2 : a1);
-      wr = rd;
-    }
+    batch_tick_coef(L, tick, flags, c, rd, wr);
     if (s < L.geo.V) {  // always true on z-shuffle lattices (V % tile == 0)
       if (!final_p) dispatch_step<T, true, SPEC>(L, ar.U, (T *)ar.P, rd, wr, c, s, mu, k0, act, k1);
       else dispatch_step<T, false, SPEC>(L, ar.U, (T *)ar.P, rd, wr, c, s, mu, k0, act, k1);

@@ -2,6 +2,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include <vector>
 
 #include "su2_launch.hpp"
 
@@ -31,6 +32,40 @@ struct BArenas {
   void *P;
 };
 
+// integrator pair k of lattice l: (P coefficient, U coefficient) in units of dtau
+__device__ inline void pair_coef(int kind, int k, double &cp, double &cu) {
+  if (kind == 6) {  // omf2 (integrator.hh:83-115): P(l) [U(1/2) P(1-2l) U(1/2) P(2l)]... P(l)
+    const double lam = 0.1938;
+    cp = (k == 0) ? lam : ((k & 1) ? 1. - 2. * lam : 2. * lam);
+    cu = 0.5;
+  } else {  // leapfrog (integrator.hh:26-50): P(1/2) U(1) [P(1) U(1)]... P(1/2)
+    cp = (k == 0) ? 0.5 : 1.0;
+    cu = 1.0;
+  }
+}
+__device__ inline double final_coef(int kind) { return kind == 6 ? 0.1938 : 0.5; }
+// tick of lattice L: the step's coefficients and the arenas it reads and writes
+__device__ inline void batch_tick_coef(const BLat &L, int tick, int flags, FusedCoef &c, int &rd,
+                                       int &wr) {
+  const int a0 = L.cur, a1 = (L.cur + 1) % 3, a2 = (L.cur + 2) % 3;
+  c.coef = L.coef;
+  c.w_t = 1.0;
+  c.w_s = 1.0;
+  c.flags = flags;
+  if (tick != L.npairs) {
+    double cp, cu;
+    pair_coef(L.kind, tick, cp, cu);
+    c.ep = cp * L.dtau;
+    c.eu = cu * L.dtau;
+    rd = (tick == 0) ? a0 : ((tick & 1) ? a1 : a2);
+    wr = (tick & 1) ? a2 : a1;
+  } else {
+    c.ep = final_coef(L.kind) * L.dtau;
+    rd = L.npairs == 0 ? a0 : (((L.npairs - 1) & 1) ? a2 : a1);
+    wr = rd;
+  }
+}
+
 // ltiles: (lattice, site_start * 4 + mu): those of the specialised SU(2)
 // lattices in d = 4 ([0, n4)), then in d = 3 ([n4, n4 + n3)), then the rest;
 // partial rows are nltiles long.  One launch per part (at most `grid` blocks
@@ -42,6 +77,22 @@ struct BArenas {
 void launch_batch_tick(int prec, const BLat *lats, const int2 *ltiles, int nltiles, int n4, int n3,
                        const BArenas &ar, int tick, int flags, double *partials, int grid,
                        int block, hipStream_t st, int only = -1, const int *active = nullptr);
+// A tick of the specialised d = 4 part with the shared-plaquette step
+// (su2_batch_plq.hip): its tiles (lattice, block of the lattice's layout) and the
+// layouts (PlqGeo, one per lattice of the batch), for the lattices `part` in that
+// order.  False where the link tiles are kept.
+struct BatchPlqPlan {
+  unsigned threads = 0, lds = 0;
+  std::vector<char> geos;
+  std::vector<int2> tiles;
+};
+bool plan_batch_plq(int prec, int ncu, const std::vector<BLat> &lat, const std::vector<size_t> &part,
+                    BatchPlqPlan &p);
+// running sites from which a tick takes it: the single lattice's line
+constexpr int batch_plq_sites(int prec) { return prec == 0 ? 32768 : 98304; }
+void launch_batch_plq(int prec, const BLat *lats, const void *geos, const int2 *tiles, int count,
+                      int rowlen, const BArenas &ar, int tick, int flags, double *partials,
+                      unsigned threads, unsigned lds, hipStream_t st);
 void launch_batch_plaq(int prec, const BLat *lats, const int2 *tiles, int ntiles, const BArenas &ar,
                        int use_final, int row, int rowlen, double *partials, int grid, int block,
                        hipStream_t st);

@@ -67,7 +67,7 @@ struct PlqGeo {
   uint32_t mnyb, mnb3;
 };
 
-// block b of nblk, thread tid -> site of the slice, chunk, row and neighbours
+// (chunk, block) pair lb, thread tid -> site of the slice, chunk, row and neighbours
 struct PlqSite {
   bool active;
   int o3;              // site within the slice
@@ -79,12 +79,9 @@ struct PlqSite {
   int lur, ldr;        // the row neighbours' thread; the halo's slot, -1 where in another block
   int luz, ldz;        // the fastest direction's neighbours' thread
 };
-__host__ __device__ __forceinline__ PlqSite plq_site(const PlqGeo &g, uint32_t b, uint32_t nblk,
-                                                     uint32_t tid, uint32_t nt) {
+__host__ __device__ __forceinline__ PlqSite plq_site_at(const PlqGeo &g, uint32_t lb, uint32_t tid,
+                                                        uint32_t nt) {
   PlqSite f;
-  // each XCD walks one contiguous eighth of the (chunk, block) sequence
-  const uint32_t xcd = b & 7u, local = b >> 3, per = nblk >> 3, rem = nblk & 7u;
-  const uint32_t lb = xcd * per + (xcd < rem ? xcd : rem) + local;
   const uint32_t chunk = fast_div(lb, g.mnb3);
   const uint32_t b3 = lb - chunk * (uint32_t)g.nb3;
   f.t0 = (int)chunk * g.Tc;
@@ -120,9 +117,15 @@ __host__ __device__ __forceinline__ PlqSite plq_site(const PlqGeo &g, uint32_t b
   }
   return f;
 }
+// the same where each XCD walks one contiguous eighth of the (chunk, block) sequence
+__host__ __device__ __forceinline__ PlqSite plq_site(const PlqGeo &g, uint32_t b, uint32_t nblk,
+                                                     uint32_t tid, uint32_t nt) {
+  const uint32_t xcd = b & 7u, local = b >> 3, per = nblk >> 3, rem = nblk & 7u;
+  return plq_site_at(g, xcd * per + (xcd < rem ? xcd : rem) + local, tid, nt);
+}
 
 inline uint32_t plq_blocks(const PlqGeo &g) { return (uint32_t)g.nb3 * (uint32_t)g.nchunk; }
-inline uint32_t plq_threads(const PlqGeo &g) {
+__host__ __device__ inline uint32_t plq_threads(const PlqGeo &g) {
   return (uint32_t)((g.rpb * g.L[g.nd - 1] + 63) / 64 * 64);
 }
 
@@ -470,19 +473,18 @@ __device__ __forceinline__ void plq_update(const typename G::link &u, const doub
 // (1 where isotropic: fma with 1 is the plain sum).  GEN: the momenta are drawn
 // (Philox counter of k_momenta_philox) instead of loaded.  NT: 0 ordinary
 // accesses, 2 non-temporal stores and momentum loads.
+// The site f of a block of nt threads; sums: this thread's part of the three.
 template <class G, int ND, bool W, bool ACC, bool GEN, int NT, class UI, class UO>
-__global__ __launch_bounds__(PLQ_NT, G::NM == 1 ? 4 : sizeof(typename G::T) == 8 ? 2 : 3) void k_md_plq(
-    UI Uin, UO Uout, const typename G::T *Pin, typename G::T *Pout, PlqGeo g, FusedCoef c,
-    double *__restrict__ partials, int pstride) {
+__device__ __forceinline__ void plq_step(const PlqSite &f, int nt, char *smem, UI Uin, UO Uout,
+                                         const typename G::T *Pin, typename G::T *Pout,
+                                         const PlqGeo &g, const FusedCoef &c, double (&sums)[3]) {
   using T = typename G::T;
   using link = typename G::link;
   using Vc = typename G::V;
   constexpr int NM = G::NM;
-  extern __shared__ __align__(16) char smem[];
-  const int nt = (int)blockDim.x, tid = (int)threadIdx.x;
+  const int tid = (int)threadIdx.x;
   constexpr int R = ND - 2, Z = ND - 1;              // row and fastest direction
   constexpr bool X4 = ND == 4;
-  const PlqSite f = plq_site(g, blockIdx.x, gridDim.x, (uint32_t)tid, (uint32_t)nt);
   const size_t V = (size_t)g.V;
   // LDS records: own, of the row above (or the halo's), of x+z; the terms' of
   // own, of the row below, of x-z
@@ -500,7 +502,6 @@ __global__ __launch_bounds__(PLQ_NT, G::NM == 1 ? 4 : sizeof(typename G::T) == 8
   const double wt = c.w_t, ws = c.w_s;
   // the action partial is the FP64 form's (FP32 takes the plaquette sum)
   constexpr bool RE = ACC && sizeof(T) == 8;
-  double sums[3] = {0.0, 0.0, 0.0};
   double re = 0.0;
 
   link own[ND], xl;
@@ -728,25 +729,46 @@ __global__ __launch_bounds__(PLQ_NT, G::NM == 1 ? 4 : sizeof(typename G::T) == 8
       s += ut;
     }
   }
+  // ReTr(U K) of every link: a plaquette's 2 Re(P) once for each of its four
+  if (ACC) sums[1] = G::RP * re;
+}
+
+// the three sums over the block's nt threads; thread k < 3 returns sum k
+__device__ __forceinline__ double plq_block_sums(const double (&sums)[3], int nt, char *smem) {
+  __syncthreads();
+  double *l3 = (double *)smem;
+  const int tid = (int)threadIdx.x, lane = tid & 63, wv = tid >> 6, nw = nt >> 6;
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    double v = sums[k];
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) v += __shfl_down(v, o, 64);
+    if (lane == 0) l3[k * 4 + wv] = v;
+  }
+  __syncthreads();
+  double v = 0.0;
+  if (tid < 3)
+    for (int i = 0; i < nw; ++i) v += l3[tid * 4 + i];
+  return v;
+}
+
+// waves per SIMD the registers are budgeted for
+template <class G> constexpr int plq_occ() {
+  return G::NM == 1 ? 4 : sizeof(typename G::T) == 8 ? 2 : 3;
+}
+
+template <class G, int ND, bool W, bool ACC, bool GEN, int NT, class UI, class UO>
+__global__ __launch_bounds__(PLQ_NT, plq_occ<G>()) void k_md_plq(
+    UI Uin, UO Uout, const typename G::T *Pin, typename G::T *Pout, PlqGeo g, FusedCoef c,
+    double *__restrict__ partials, int pstride) {
+  extern __shared__ __align__(16) char smem[];
+  const int nt = (int)blockDim.x;
+  const PlqSite f = plq_site(g, blockIdx.x, gridDim.x, threadIdx.x, (uint32_t)nt);
+  double sums[3] = {0.0, 0.0, 0.0};
+  plq_step<G, ND, W, ACC, GEN, NT>(f, nt, smem, Uin, Uout, Pin, Pout, g, c, sums);
   if (ACC) {
-    // ReTr(U K) of every link: a plaquette's 2 Re(P) once for each of its four
-    sums[1] = G::RP * re;
-    __syncthreads();
-    double *l3 = (double *)smem;
-    const int lane = tid & 63, wv = tid >> 6, nw = nt >> 6;
-#pragma unroll
-    for (int k = 0; k < 3; ++k) {
-      double v = sums[k];
-#pragma unroll
-      for (int o = 32; o > 0; o >>= 1) v += __shfl_down(v, o, 64);
-      if (lane == 0) l3[k * 4 + wv] = v;
-    }
-    __syncthreads();
-    if (tid < 3) {
-      double v = 0.0;
-      for (int i = 0; i < nw; ++i) v += l3[tid * 4 + i];
-      partials[(size_t)tid * pstride + blockIdx.x] = v;
-    }
+    const double v = plq_block_sums(sums, nt, smem);
+    if (threadIdx.x < 3) partials[(size_t)threadIdx.x * pstride + blockIdx.x] = v;
   }
 }
 
