@@ -1408,7 +1408,7 @@ int su2gpu_sweep(su2gpu_lattice *h, uint64_t seed, uint64_t sweep, double delta,
       {
         Prof pr(h, "sweep");
         su2k::launch_sweep(h->group, h->prec, h->U[h->cur], h->geo, mu, par, list, nlist, seed,
-                           sweep, delta, (int)n_hit, h->beta / Nc(h), w_t, w_s, h->aniso ? 1 : 0,
+                           sweep, delta, (int)n_hit, h->beta / Nc(h), w_t, w_s,
                            row(h, r), h->stream);
       }
       CK(last_launch("sweep"));

@@ -133,7 +133,7 @@ void launch_flow_stage_adj(int prec, const void *Zs, void *lamW, void *lamZ, int
 int sweep_blocks(const Geo &g, int nlist);  // nlist < 0: the parity form
 void launch_sweep(int group, int prec, void *U, const Geo &g, int mu, int parity, const int *list,
                   int nlist, uint64_t seed, uint64_t sweep, double delta, int n_hit,
-                  double beta_nc, double w_t, double w_s, int aniso, double *partials,
+                  double beta_nc, double w_t, double w_s, double *partials,
                   hipStream_t st);
 // lamW += b (dD/dW)^T lamZ; R: scratch of 36 V reals (the b and c role
 // gradients of the 6 planes).  gather = false leaves the R terms to a later

@@ -82,13 +82,19 @@ __device__ __forceinline__ bool below_exp(double v, double dS) {
 }
 
 // What bounds it: at one hit the link gathers (every second site of a row: half
-// of each line a wave touches, 0.5 of the 0.68 ms of an FP64 32^4 sweep of 10
-// hits), beyond a few hits the vector units.  Against blocks dealt round the XCDs,
-// one direction at run time (a round trip per plane) and the library's sincospi,
-// sqrt, exp and division: FP64 32^4 10 hits 679 -> 520 us, 1 hit 517 -> 411 us, FP32
-// 570 -> 450 and 281 -> 218 us, U(1) 24^4 FP64 201 -> 153 us, three colours (15 21 7
-// 32) 168 -> 146 us.  With 4 waves per SIMD (128 registers); 3, 5 and 6: 520, 525,
-// 565 us.
+// of each line a wave touches; 155 to 195 MB from beyond the L2 per launch of FP64
+// 32^4), beyond a few hits the vector units.  Against blocks dealt round the XCDs,
+// one direction at run time, coordinates by division, a branch on the weights
+// between the planes' loads and the library's sincospi, sqrt, exp and division: FP64
+// 32^4 10 hits 679 -> 520 us, 1 hit 517 -> 411 us, FP32 570 -> 418 and 281 -> 178 us,
+// U(1) 24^4 FP64 201 -> 149 us, 8^4 1 hit 65 -> 60 us (before the last two of these:
+// FP32 450 and 218, U(1) 153), three colours (15 21 7 32) 168 -> 146 us.
+//
+// FP64 SU(2), records of 32 bytes: the loads of one plane at a time (all of a side's
+// take 128 registers and 20 spills: 619 us) and at most 4 blocks on a CU, held
+// by SWEEP_PAD bytes of LDS: with the 7 that the registers allow the blocks' lines
+// push each other out of the L2, 550 against 526 us (5 and 3 blocks: 535, 553).
+constexpr unsigned SWEEP_PAD = 40 * 1024 - 64;
 // list == nullptr: the sites of parity `parity` (every extent even);
 // otherwise the nlist sites list[0 .. nlist) of one colour class
 template <class G, int ND, int mu>
@@ -96,7 +102,7 @@ __global__ __launch_bounds__(NTS, 4) void k_sweep(typename G::link *__restrict__
                                                int parity, const int *__restrict__ list,
                                                int nlist, uint64_t seed, uint64_t sweep,
                                                double delta, int n_hit, double beta_nc,
-                                               double w_t, double w_s, int aniso,
+                                               double w_t, double w_s,
                                                double *__restrict__ partials) {
   using T = typename G::real;
   using link = typename G::link;
@@ -115,45 +121,69 @@ __global__ __launch_bounds__(NTS, 4) void k_sweep(typename G::link *__restrict__
   const int j = lb * NTS + threadIdx.x;
   double accepted = 0.0;
   if (list ? j < nlist : j < V / 2) {
-    int s;
+    int s, up[ND], dn[ND];
     if (list) {
       s = list[j];
+      neighbour_offsets<ND>(geo, s, up, dn);
     } else {
-      // site j of this parity: row of the fastest direction, then every second site
-      const int Lf = geo.L[ND - 1];  // fastest direction in use (even)
-      const int half = Lf / 2;
-      const int row = j / half, k = j - row * half;
-      int rp = 0, q = row;
+      // site j of this parity: pair j of neighbours along the fastest direction
+      // (even), and of the two the one with that parity
+      int c[ND], rp = 0;
+      uint32_t q = 2u * (uint32_t)j;
 #pragma unroll
-      for (int d = ND - 2; d >= 0; --d) {
-        const int Ld = geo.L[d];
-        const int qn = q / Ld;
-        rp += q - qn * Ld;
+      for (int d = ND - 1; d > 0; --d) {
+        const uint32_t Ld = (uint32_t)geo.L[d];
+        const uint32_t qn = geo.fdiv ? (geo.mL[d] ? __umulhi(q, geo.mL[d]) : q) : q / Ld;
+        c[d] = (int)(q - qn * Ld);
         q = qn;
+        if (d < ND - 1) rp += c[d];
       }
-      s = row * Lf + 2 * k + ((parity + rp) & 1);
+      c[0] = (int)q;
+      rp += c[0];
+      const int odd = (parity + rp) & 1;
+      c[ND - 1] += odd;
+      s = 2 * j + odd;
+#pragma unroll
+      for (int d = 0; d < ND; ++d) {
+        up[d] = c[d] == geo.L[d] - 1 ? -(geo.L[d] - 1) * geo.str[d] : geo.str[d];
+        dn[d] = c[d] == 0 ? (geo.L[d] - 1) * geo.str[d] : -geo.str[d];
+      }
     }
-    int up[ND], dn[ND];
-    neighbour_offsets<ND>(geo, s, up, dn);
-    // staples (get_staples.hh:26-80): all upper, then all lower
+    // staples (get_staples.hh:26-80): all upper, then all lower; the weights are 1
+    // on an isotropic lattice (a branch round each product would keep the next
+    // plane's loads behind it)
     acc K = G::zero();
+    link u = U[mu * V + s];
+    // one round trip for the links of a side's planes, one for each plane where
+    // they are records of 32 bytes
+    constexpr bool EACH = sizeof(link) > 16;
 #pragma unroll
-    for (int nu = 0; nu < ND; ++nu) {
-      if (nu == mu) continue;
-      acc t = G::upper(U[nu * V + s + up[mu]], U[mu * V + s + up[nu]], U[nu * V + s]);
-      if (aniso) t = G::scale(T((mu == 0 || nu == 0) ? w_t : w_s), t);
-      K = G::add(K, t);
-    }
+    for (int side = 0; side < 2; ++side) {
+      link l[3 * ND];
+      auto fetch = [&](int nu) {
+        const int o = side == 0 ? 0 : dn[nu];
+        l[3 * nu] = U[nu * V + s + up[mu] + o];
+        l[3 * nu + 1] = U[mu * V + s + (side == 0 ? up[nu] : o)];
+        l[3 * nu + 2] = U[nu * V + s + o];
+      };
+      if constexpr (!EACH) {
 #pragma unroll
-    for (int nu = 0; nu < ND; ++nu) {
-      if (nu == mu) continue;
-      acc t = G::lower(U[nu * V + s + up[mu] + dn[nu]], U[mu * V + s + dn[nu]],
-                       U[nu * V + s + dn[nu]]);
-      if (aniso) t = G::scale(T((mu == 0 || nu == 0) ? w_t : w_s), t);
-      K = G::add(K, t);
+        for (int nu = 0; nu < ND; ++nu)
+          if (nu != mu) fetch(nu);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+#pragma unroll
+      for (int nu = 0; nu < ND; ++nu) {
+        if (nu == mu) continue;
+        if (EACH) fetch(nu);
+        const acc t = side == 0 ? G::upper(l[3 * nu], l[3 * nu + 1], l[3 * nu + 2])
+                                : G::lower(l[3 * nu], l[3 * nu + 1], l[3 * nu + 2]);
+        K = G::add(K, G::scale(T((mu == 0 || nu == 0) ? w_t : w_s), t));
+        if (EACH) __builtin_amdgcn_sched_barrier(0);
+      }
+      __builtin_amdgcn_sched_barrier(0);
     }
     const uint32_t lid = (uint32_t)s * (uint32_t)ND + (uint32_t)mu;
-    link u = U[mu * V + s];
     // ReTr(u K), kept from hit to hit
     [[maybe_unused]] double retr;
     [[maybe_unused]] quat<double> Kd;
@@ -213,13 +243,13 @@ int sweep_blocks(const Geo &g, int nlist) { return ((nlist >= 0 ? nlist : g.V / 
 template <class G, int ND>
 static void sweep_nd(void *U, const Geo &g, int mu, int parity, const int *list, int nlist,
                      uint64_t seed, uint64_t sweep, double delta, int n_hit, double beta_nc,
-                     double w_t, double w_s, int aniso, double *partials, hipStream_t st) {
+                     double w_t, double w_s, double *partials, hipStream_t st) {
   using link = typename G::link;
   const dim3 grid(sweep_blocks(g, list ? nlist : -1));
   if (grid.x == 0) return;
 #define SU2_SWEEP(M)                                                                          \
-  hipLaunchKernelGGL((k_sweep<G, ND, M>), grid, dim3(NTS), 0, st, (link *)U, g, parity, list, \
-                     nlist, seed, sweep, delta, n_hit, beta_nc, w_t, w_s, aniso, partials)
+  hipLaunchKernelGGL((k_sweep<G, ND, M>), grid, dim3(NTS), sizeof(link) > 16 ? SWEEP_PAD : 0, st, (link *)U,    \
+                     g, parity, list, nlist, seed, sweep, delta, n_hit, beta_nc, w_t, w_s, partials)
   if (mu == 0) SU2_SWEEP(0);
   else if (mu == 1) SU2_SWEEP(1);
   else if (ND > 2 && mu == 2) SU2_SWEEP((ND > 2 ? 2 : 0));
@@ -229,9 +259,9 @@ static void sweep_nd(void *U, const Geo &g, int mu, int parity, const int *list,
 
 void launch_sweep(int group, int prec, void *U, const Geo &g, int mu, int parity, const int *list,
                   int nlist, uint64_t seed, uint64_t sweep, double delta, int n_hit,
-                  double beta_nc, double w_t, double w_s, int aniso, double *partials,
+                  double beta_nc, double w_t, double w_s, double *partials,
                   hipStream_t st) {
-#define SWEEP_ARGS U, g, mu, parity, list, nlist, seed, sweep, delta, n_hit, beta_nc, w_t, w_s, aniso, partials, st
+#define SWEEP_ARGS U, g, mu, parity, list, nlist, seed, sweep, delta, n_hit, beta_nc, w_t, w_s, partials, st
 #define SWEEP_G(G)                               \
   do {                                           \
     if (g.nd == 2) sweep_nd<G, 2>(SWEEP_ARGS);   \
