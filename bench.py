@@ -440,43 +440,26 @@ def progress(msg):
 
 
 def kernel_name(prec, L):
-    """Instantiation of the specialised step that a P-then-U launch of the
-    L^4 SU(2) lattice takes (su2_kernels.hip launch_fast), as rocprofv3 names
-    it: <T, WRITE_U, ACCUM, SPEC, ZS, AN, NT, link in, link out>.  ZS: 1 the
-    +-z lane exchange within a wave (64 % L == 0), 2 the general exchange
-    (FP32 beyond 256 MiB otherwise), 0 none.  NT: non-temporal stores (1)
-    and momentum loads (2: the FP32 general-exchange step, both forms with the
-    lane exchange or in FP64 beyond 1 GiB) where the two link fields and the
-    momenta exceed 256 MiB.
-    The FP64 form steps on the half-field layout (QHalf in, QHalfW out); with
-    >= 4 t-slices per XCD the step is a t-walk: FP64 with the lane exchange
-    k_md_su2_4d_tww<T, NT, in, out> (one direction per wave; beyond 1 GiB of
-    fields k_md_su2_4d_tw), FP32 with it (within the Infinity Cache)
-    k_md_su2_4d_tw<T, ZS, NT, in, out>, and with the general exchange
-    k_md_su2_4d_twz<T, NT, in, out>."""
+    """Instantiation of the step that a P-then-U launch of the L^4 SU(2) lattice
+    takes, as rocprofv3 names it.  From 32768 (FP64) or 98304 sites (FP32) and up
+    to rows of 128: k_md_plq<group, nd, write U, sums, draw, NT, link in, link out>
+    (su2_plq.hip), non-temporal (NT = 2) where the two link fields and the momenta
+    exceed 256 MiB; FP64 on the half-field layout where the 3-volume is a
+    multiple of 256.  Below: k_md_su2_4d<T, WRITE_U, ACCUM, SPEC, ZS, AN, NT, in,
+    out> (su2_md_fast.hpp) on the same condition, ZS = 1 with the +-z lane exchange
+    (64 % L == 0); else the general steps k_md_link (FP64) and k_md_su2_geo (FP32)."""
     r = 8 if prec == 0 else 4
-    big = 4 * L ** 4 * (2 * 4 * r + 3 * r) > 256 * 1024 * 1024
-    if prec == 0:
+    t = "double" if prec == 0 else "float"
+    nt = 2 if 4 * L ** 4 * (2 * 4 * r + 3 * r) > 256 * 1024 * 1024 else 0
+    half = prec == 0 and L ** 3 % 256 == 0
+    link = ("su2k::QHalf, su2k::QHalfW" if half
+            else f"su2dev::quat<{t}> const*, su2dev::quat<{t}>*")
+    if L ** 4 >= (32768 if prec == 0 else 98304) and L <= 128:
+        return f"k_md_plq<su2k::PlqSU2<{t}>, 4, true, false, false, {nt}, {link}>"
+    if L ** 3 % 256 == 0:
         zs = 1 if 64 % L == 0 else 0
-        nt = (2 if 4 * L ** 4 * (2 * 4 * r + 3 * r) > 1024 ** 3 else 1) if big else 0
-        if zs == 1 and L % 8 == 0 and L // 8 >= 4:
-            if nt < 2:
-                return f"k_md_su2_4d_tww<double, {nt}, su2k::QHalf, su2k::QHalfW>"
-            return f"k_md_su2_4d_tw<double, 1, {nt}, su2k::QHalf, su2k::QHalfW>"
-        if zs == 0 and L % 8 == 0 and L // 8 >= 4:
-            return f"k_md_su2_4d_twz<double, {nt}, su2k::QHalf, su2k::QHalfW>"
-        return f"k_md_su2_4d<double, true, false, 1, {zs}, false, {nt}, su2k::QHalf, su2k::QHalfW>"
-    zs = 1 if 64 % L == 0 else (2 if big else 0)
-    huge = 4 * L ** 4 * (2 * 4 * r + 3 * r) > 1024 ** 3
-    nt = (2 if zs == 2 or (zs == 1 and huge) else 1) if big else 0
-    if zs == 1 and not big and L % 8 == 0 and L // 8 >= 4:
-        # the t-walk: each thread walks the t-slices of its XCD's chunk
-        return "k_md_su2_4d_tw<float, 1, 0, su2dev::quat<float> const*, su2dev::quat<float>*>"
-    if zs == 2 and L % 8 == 0 and L // 8 >= 4:
-        # the t-walk with the general exchange, one direction per wave
-        return "k_md_su2_4d_twz<float, 2, su2dev::quat<float> const*, su2dev::quat<float>*>"
-    return (f"k_md_su2_4d<float, true, false, 1, {zs}, false, {nt}, su2dev::quat<float> const*, "
-            "su2dev::quat<float>*>")
+        return f"k_md_su2_4d<{t}, true, false, 1, {zs}, false, 0, {link}>"
+    return "k_md_link" if prec == 0 else "k_md_su2_geo"
 
 
 def form_roofline(f, prec, L):

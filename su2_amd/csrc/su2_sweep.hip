@@ -82,8 +82,9 @@ __device__ __forceinline__ bool below_exp(double v, double dS) {
 }
 
 // What bounds it: at one hit the link gathers (every second site of a row: half
-// of each line a wave touches; 155 to 195 MB from beyond the L2 per launch of FP64
-// 32^4), beyond a few hits the vector units.  Against blocks dealt round the XCDs,
+// of each line a wave touches; a launch of FP64 32^4 fetches 310 to 390 MB from beyond
+// the L2, 2.3 to 2.9 times the field, at 6.5 TB/s with one hit and 5.5 with 10),
+// beyond a few hits the vector units.  Against blocks dealt round the XCDs,
 // one direction at run time, coordinates by division, a branch on the weights
 // between the planes' loads and the library's sincospi, sqrt, exp and division: FP64
 // 32^4 10 hits 679 -> 520 us, 1 hit 517 -> 411 us, FP32 570 -> 418 and 281 -> 178 us,
