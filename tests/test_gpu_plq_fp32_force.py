@@ -1,0 +1,71 @@
+"""The FP32 force of the shared-plaquette step keeps the precision of the staple
+steps: FP32 staples of two products each, summed and projected in FP64.
+
+That arithmetic is replayed here on the host (an FP32 FMA is the FP64 fused value
+rounded once, to within double rounding), and the step's rms error against the FP64
+force of the same links may exceed the replay's by 5 %: at 4e5 force components the
+rms is known to 0.2 %, and the step associates its products differently, which
+moves it by a few per cent.  A force projected in FP32 is 16 % and more above."""
+import numpy as np
+import pytest
+
+import su2_amd as S
+
+pytestmark = pytest.mark.gpu
+
+
+def _fma(a, b, c):
+    return (a.astype(np.float64) * b.astype(np.float64) + c).astype(np.float32)
+
+
+def _mul(u, v):
+    f = _fma
+    return np.stack([
+        f(u[0], v[0], -f(u[1], v[1], f(u[2], v[2], u[3] * v[3]))),
+        f(u[0], v[1], f(u[1], v[0], f(-u[3], v[2], u[2] * v[3]))),
+        f(u[0], v[2], f(-u[1], v[3], f(u[2], v[0], u[3] * v[1]))),
+        f(u[0], v[3], f(u[1], v[2], f(u[3], v[0], -(u[2] * v[1]))))])
+
+
+def _dag(u):
+    return np.stack([u[0], -u[1], -u[2], -u[3]])
+
+
+def _replay(U, dims, xi):
+    """2 Im(U K), staples in FP32, sums and projection in FP64: (V, nd, 3)"""
+    Lx, Ly, Lz, Lt, nd = dims
+    shape = (Lt, Lx, Ly, Lz)[:nd]
+    q = [np.moveaxis(U.reshape(shape + (nd, 4))[..., m, :], -1, 0).astype(np.float32)
+         for m in range(nd)]
+    up = lambda a, d: np.roll(a, -1, d + 1)  # noqa: E731
+    dn = lambda a, d: np.roll(a, 1, d + 1)  # noqa: E731
+    out = []
+    for mu in range(nd):
+        K = 0.0
+        for nu in range(nd):
+            if nu == mu:
+                continue
+            w = 1.0 / xi if 0 in (mu, nu) else xi
+            a = _mul(_mul(up(q[nu], mu), _dag(up(q[mu], nu))), _dag(q[nu]))
+            b = dn(_mul(_mul(_dag(up(q[nu], mu)), _dag(q[mu])), q[nu]), nu)
+            K = K + w * (a.astype(np.float64) + b.astype(np.float64))
+        u = q[mu].astype(np.float64)
+        ai = u[0] * K[1] + u[1] * K[0] - u[3] * K[2] + u[2] * K[3]
+        br = u[0] * K[2] - u[1] * K[3] + u[2] * K[0] + u[3] * K[1]
+        bi = u[0] * K[3] + u[1] * K[2] + u[3] * K[0] - u[2] * K[1]
+        out.append(2.0 * np.stack([bi, br, ai], -1))
+    return np.stack(out, -2).reshape(-1, 3)
+
+
+@pytest.mark.parametrize("dims,xi", [((24, 16, 18, 16, 4), 1.0), ((16, 16, 32, 17, 4), 1.7),
+                                     ((64, 32, 1, 64, 3), 1.0)])
+def test_fp32_force_error(oracle, dims, xi):
+    U = oracle.hotstart(1, dims, 20251, 0.4).astype(np.float32).astype(np.float64)
+    exact = oracle.derivative(1, dims, U, 2.0, xi=xi).reshape(-1, 3)  # beta / Nc = 1
+    want = _replay(U, dims, xi).astype(np.float32) - exact
+    with S.Lattice(S.SU2, dims, 2.0, xi=xi, precision=S.FP32) as lat:
+        lat.set_links(U)
+        got = lat.derivative(1.0).reshape(-1, 3) - exact
+    rms = lambda x: float(np.sqrt((x * x).mean()))  # noqa: E731
+    print(dims, xi, "rms error", rms(got), "replay", rms(want))
+    assert rms(got) < 1.05 * rms(want)
