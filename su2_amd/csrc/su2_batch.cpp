@@ -19,6 +19,7 @@
 
 #include "../../include/su2_mi355x.h"
 #include "su2_batch.hpp"
+#include "su2_pinned.hpp"
 
 namespace su2k {
 void launch_links_from_aos(int group, int prec, const double *src, int stride, int offset,
@@ -399,25 +400,10 @@ int ensure_stage(B *b, size_t n) {
   return SU2GPU_OK;
 }
 
-// the device address of a pinned host range, or null: a download of up to
-// DIRECT_BYTES goes there straight from the kernel that converts it, without
+// a download of up to DIRECT_BYTES into pinned memory goes there straight from the kernel that converts it, without
 // a staging copy (the 224 members of the mixed ensemble, 173 MB in all: 8.2 -> 6.0
 // ms, 3.3 at the link's rate); larger ones, and pageable memory, are staged
 constexpr size_t DIRECT_BYTES = 4 << 20;
-double *pinned_on_device(double *p, size_t bytes) {
-  if (bytes > DIRECT_BYTES) return nullptr;
-  hipPointerAttribute_t a, z;
-  if (hipPointerGetAttributes(&a, p) != hipSuccess ||
-      hipPointerGetAttributes(&z, (char *)p + bytes - 1) != hipSuccess) {
-    (void)hipGetLastError();  // pageable memory: not an error here
-    return nullptr;
-  }
-  if (a.type != hipMemoryTypeHost || z.type != hipMemoryTypeHost || !a.devicePointer || !z.devicePointer)
-    return nullptr;
-  // both ends in one mapping
-  if ((char *)z.devicePointer - (char *)a.devicePointer != (ptrdiff_t)(bytes - 1)) return nullptr;
-  return (double *)a.devicePointer;
-}
 
 std::string signature(const B *b) {
   std::ostringstream ss;
@@ -578,7 +564,7 @@ int su2gpu_batch_get_links(su2gpu_batch *b, size_t i, double *dst) {
   const int nc = L.group == 1 ? 4 : 1;
   const size_t n = (size_t)L.geo.V * L.geo.nd * nc;
   // a pinned destination: the conversion kernel writes there itself
-  double *to = pinned_on_device(dst, n * sizeof(double));
+  double *to = n * sizeof(double) > DIRECT_BYTES ? nullptr : su2k::pinned_on_device(dst, n * sizeof(double));
   if (!to) BK(ensure_stage(b, n));
   su2k::launch_links_to_aos(L.group, b->prec, b->ar.U[L.cur] + L.uoff, to ? to : b->staging, nc, 0,
                             L.geo.V, L.geo.nd, b->stream);
