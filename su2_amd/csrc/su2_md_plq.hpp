@@ -299,11 +299,17 @@ template <> struct PlqSU2<float> {
   }
 };
 
-// sin and cos of t = q pi/2 + r, |r| <= pi/4 (pi/2 in two parts, the first of
-// 33 bits, so that q times it is exact for the q < 2^17 that occur), by Taylor
-// series in r^2 to the eighth power (remainders below 1e-18)
-__device__ __forceinline__ void plq_series(double y, double &c, double &s) {
-  double t = fma(y, 1.0 / 20922789888000.0, -1.0 / 87178291200.0);
+// sin and cos of t = q pi/2 + r, |r| <= pi/4 (Cody and Waite, Software Manual for the
+// Elementary Functions, 1980: pi/2 in two parts, the first its leading 33 bits, so that
+// q times it is exact for the q < 2^17 that occur, the second the rest rounded), by
+// Taylor series to the eighth power of y = r^2: cos r = c, sin r = r + r y w.  First
+// terms left out, at y = (pi/4)^2: 2.1e-18 of the cosine, 1.1e-19 of the sine's.  LONG:
+// the cosine's ninth power too (at y = 1 the first terms left out are 4e-19 and 8e-18).
+template <bool LONG = false>
+__host__ __device__ __forceinline__ void plq_series(double y, double &c, double &w) {
+  double t = 1.0 / 20922789888000.0;
+  if (LONG) t = fma(y, -1.0 / 6402373705728000.0, t);
+  t = fma(y, t, -1.0 / 87178291200.0);
   double u = fma(y, 1.0 / 355687428096000.0, -1.0 / 1307674368000.0);
   t = fma(y, t, 1.0 / 479001600);
   u = fma(y, u, 1.0 / 6227020800.0);
@@ -318,15 +324,21 @@ __device__ __forceinline__ void plq_series(double y, double &c, double &s) {
   t = fma(y, t, -0.5);
   u = fma(y, u, -1.0 / 6);
   c = fma(y, t, 1.0);
-  s = fma(y, u, 1.0);
+  w = u;
 }
-__device__ __forceinline__ double plq_reduce(double a, int &j) {
+__host__ __device__ __forceinline__ void plq_sincos(double r, double &c, double &s) {
+  const double y = r * r;
+  double w;
+  plq_series(y, c, w);
+  s = fma(r * y, w, r);
+}
+__host__ __device__ __forceinline__ double plq_reduce(double a, int &j) {
   if (fabs(a) > 1e5) a = fmod(a, 6.283185307179586477);
   const double q = rint(a * 0.6366197723675813431);
   j = (int)q;
   return fma(-q, 6.07710050650619224932e-11, fma(-q, 1.57079632673412561417, a));
 }
-__device__ __forceinline__ void plq_quadrant(int j, double &c, double &s) {
+__host__ __device__ __forceinline__ void plq_quadrant(int j, double &c, double &s) {
   const double sn = (j & 1) ? c : s, cs = (j & 1) ? s : c;
   c = ((j + 1) & 2) ? -cs : cs;
   s = (j & 2) ? -sn : sn;
@@ -354,8 +366,7 @@ template <typename T_> struct PlqU1 {
       int j;
       const double r = plq_reduce(th, j);
       double cs, sn;
-      plq_series(r * r, cs, sn);
-      sn *= r;
+      plq_sincos(r, cs, sn);
       plq_quadrant(j, cs, sn);
       if (RE) co = cs;
       return sn;
@@ -458,22 +469,23 @@ template <typename T, int N> __device__ __forceinline__ void plq_pin(T (&v)[N]) 
   for (int k = 0; k < N; ++k) asm volatile("" : "+v"(v[k]));
 }
 
-// cos a and sin(a)/a of the FP64 update for x = a^2: the series in x where
-// x <= 1 (remainders x^9 / 18! <= 1.6e-16 and x^9 / 19!), beyond that in the
-// square of the reduced angle
-__device__ __forceinline__ void cos_sinc_fp64(double x, double &c, double &s) {
-  double y = x, r = 0.0;
+// cos a and sin(a)/a of the FP64 update for x = a^2: the series in x up to 1, beyond
+// that in the square of the reduced angle
+__host__ __device__ __forceinline__ void cos_sinc_fp64(double x, double &c, double &s) {
+  double y = x, r = 0.0, w;
   int j = 0;
   const bool big = !(x <= 1.0);
   if (big) {
     r = plq_reduce(sqrt(x), j);
     y = r * r;
   }
-  plq_series(y, c, s);
+  plq_series<true>(y, c, w);
   if (big) {
-    s *= r;
+    s = fma(r * y, w, r);
     plq_quadrant(j, c, s);
     s = s / sqrt(x);
+  } else {
+    s = fma(y, w, 1.0);
   }
 }
 

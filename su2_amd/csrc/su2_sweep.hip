@@ -47,14 +47,13 @@ __device__ __forceinline__ double retr_mul_u1(double th, double kre, double kim)
   return c * kre - s * kim;
 }
 
-// sin(pi x) and cos(pi x): r = x - q / 2 exact, |r| <= 1/4, then the Taylor
-// series of both in (pi r)^2 <= 0.62 (remainders below 1e-18)
+// sin(pi x) and cos(pi x), |x| < 2^30: r = x - q / 2 exact, |r| <= 1/4, then the
+// Taylor series of both in (pi r)^2 <= 0.62 (first terms left out below 2.1e-18)
 __device__ __forceinline__ void sincospi_series(double x, double *sn, double *cs) {
   const double q = rint(2.0 * x);
   const double r = M_PI * fma(-0.5, q, x);
   double c, s;
-  plq_series(r * r, c, s);
-  s *= r;
+  plq_sincos(r, c, s);
   plq_quadrant((int)q, c, s);
   *sn = s;
   *cs = c;
@@ -205,7 +204,9 @@ __global__ __launch_bounds__(NTS, 4) void k_sweep(typename G::link *__restrict__
         const double uu = -1.0 + 2.0 * u01_32(c[1]);
         const double r = sqrt_unit(1.0 - uu * uu);
         double sa, ca, st, ct;
-        sincospi_series(2.0 * delta * u01_32(c[0]), &sa, &ca);
+        double x = 2.0 * delta * u01_32(c[0]);
+        if (fabs(delta) > 1e6) x = fma(-2.0, rint(0.5 * x), x);  // a whole number of turns off
+        sincospi_series(x, &sa, &ca);
         sincospi_series(2.0 * u01_32(c[2]), &st, &ct);
         const quat<double> R{ca, sa * uu, sa * r * st, sa * r * ct};
         const quat<double> ud = to_d(u);
