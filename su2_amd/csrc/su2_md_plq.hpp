@@ -175,20 +175,19 @@ inline bool make_plq_rows(const int L[4], int nd, int V, PlqGeo &g, int threads 
 // the slice below it).
 inline bool make_plq_chunks(int percu, int cus, PlqGeo &g) {
   const int waves = (g.rpb * g.L[g.nd - 1] + 63) / 64;
+  const long round = (long)percu * cus;
   double cost = 1e300;
   g.Tc = 1;
   for (int Tc = 1; Tc <= g.L[0]; ++Tc) {
-    const int nc = (g.L[0] + Tc - 1) / Tc;
-    double c = 0.0;
-    for (long left = (long)g.nb3 * nc; left > 0; left -= (long)percu * cus) {
-      const long b = std::min<long>((left + cus - 1) / cus, percu);
-      c += (Tc + 0.35) * (2.0 + (double)(b * waves));
-      if (c > cost) break;
-    }
+    const long nb = (long)g.nb3 * ((g.L[0] + Tc - 1) / Tc), full = (nb - 1) / round;
+    const long last = (nb - full * round + cus - 1) / cus;
+    const double c =
+        (Tc + 0.35) * ((double)full * (2.0 + percu * waves) + 2.0 + (double)(last * waves));
     if (c < cost * 0.999) {
       cost = c;
       g.Tc = Tc;
     }
+    if (nb <= cus) break;  // one block on some of the CUs: longer chunks only cost more
   }
   g.nchunk = (g.L[0] + g.Tc - 1) / g.Tc;
   if ((uint64_t)g.nb3 * g.nchunk * g.nb3 >= (1ull << 32)) return false;
