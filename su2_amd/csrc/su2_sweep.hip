@@ -23,6 +23,8 @@
 // its words give alpha, u, theta and the acceptance uniform, each as
 // (word + 1/2) 2^-32.  The chain therefore depends on (seed, sweep number) only,
 // not on the launch shape; it is not the reference's per-thread mt19937 stream.
+#include <algorithm>
+
 #include "su2_device.hpp"
 #include "su2_launch.hpp"
 #include "su2_md_plq.hpp"
@@ -93,13 +95,16 @@ __device__ __forceinline__ bool below_exp(double v, double dS) {
 // FP64 SU(2), records of 32 bytes: the loads of one plane at a time (all of a side's
 // take 128 registers and 20 spills: 619 us) and at most 4 blocks on a CU, held
 // by SWEEP_PAD bytes of LDS: with the 7 that the registers allow the blocks' lines
-// push each other out of the L2, 550 against 526 us (5 and 3 blocks: 535, 553).
+// push each other out of the L2, 550 against 526 us (5 and 3 blocks: 535, 553).  The cap
+// was not slower at any size tried (with / without): 16^4 one hit 65.9 / 67.6, 48^4 one hit
+// 2176 / 2205, ten 2286 / 2474, d = 3 96^3 188 / 198 and 300 / 304, 128^3 532 / 551, d = 2 2048^2
+// 282 / 286, three colours 33^4 741 / 750 us.
 constexpr unsigned SWEEP_PAD = 40 * 1024 - 64;
 // list == nullptr: the sites of parity `parity` (every extent even);
 // otherwise the nlist sites list[0 .. nlist) of one colour class
 template <class G, int ND, int mu>
 __global__ __launch_bounds__(NTS, 4) void k_sweep(typename G::link *__restrict__ U, Geo geo,
-                                               int parity, const int *__restrict__ list,
+                                               int parity, int tw, const int *__restrict__ list,
                                                int nlist, uint64_t seed, uint64_t sweep,
                                                double delta, int n_hit, double beta_nc,
                                                double w_t, double w_s,
@@ -109,14 +114,11 @@ __global__ __launch_bounds__(NTS, 4) void k_sweep(typename G::link *__restrict__
   using acc = typename G::acc;
   __shared__ double lds[NTS / 64];
   const int V = geo.V;
-  // each XCD walks one contiguous eighth of the sites; where the t slices divide
-  // into eighths and into blocks, with t fastest, so that a block's t neighbours
-  // were fetched by the blocks just before it into the same L2
   int lb = xcd_block(blockIdx.x, gridDim.x);
-  if (!list && geo.L[0] % 8 == 0 && (V / 2 / geo.L[0]) % NTS == 0) {
+  if (tw > 0) {
     const int nb3 = V / 2 / geo.L[0] / NTS, Tc = geo.L[0] / 8;
-    const int l = blockIdx.x >> 3, q = l / Tc;
-    lb = ((int)(blockIdx.x & 7) * Tc + l - q * Tc) * nb3 + q;
+    const int l = blockIdx.x >> 3, w = l / (tw * nb3), r = l - w * tw * nb3, q = r / tw;
+    lb = ((int)(blockIdx.x & 7) * Tc + w * tw + r - q * tw) * nb3 + q;
   }
   const int j = lb * NTS + threadIdx.x;
   double accepted = 0.0;
@@ -240,6 +242,23 @@ __global__ __launch_bounds__(NTS, 4) void k_sweep(typename G::link *__restrict__
   if (threadIdx.x == 0) partials[lb] = r;
 }
 
+// The order of the blocks.  Each XCD walks one contiguous eighth of the sites.  Where
+// the t slices divide into eighths and into blocks (tw > 0), it walks them in groups of
+// tw slices, t fastest within a group, so that a block's t neighbours were fetched by
+// the blocks just before it into the same L2.  Groups of 4 to 7 slices: slices lie a
+// whole number of L2 ways apart where the extents are powers of two, and then eight or
+// more of them push each other out (FP64, one hit, groups of 4 / 8 / all slices / memory
+// order: 128^3 d = 3 415 / 486 / 530 / 430 us, 32^3 x 128 1667 / 1911 / 2081 / 1872, 64^4 6786 /
+// 7453 / 7453 / 7834); elsewhere longer groups are as good (40^4 in 5 1043, memory order
+// 1189; 48^4 in 6 2176, in 3 2206, memory order 2433 us).
+static int sweep_tw(const Geo &g) {
+  if (g.L[0] % 8 != 0 || (g.V / 2 / g.L[0]) % NTS != 0) return 0;
+  const int Tc = g.L[0] / 8;
+  int tw = std::min(Tc, 7);
+  while (Tc % tw != 0) --tw;
+  return tw;
+}
+
 int sweep_blocks(const Geo &g, int nlist) { return ((nlist >= 0 ? nlist : g.V / 2) + NTS - 1) / NTS; }
 
 template <class G, int ND>
@@ -251,7 +270,7 @@ static void sweep_nd(void *U, const Geo &g, int mu, int parity, const int *list,
   if (grid.x == 0) return;
 #define SU2_SWEEP(M)                                                                          \
   hipLaunchKernelGGL((k_sweep<G, ND, M>), grid, dim3(NTS), sizeof(link) > 16 ? SWEEP_PAD : 0, st, (link *)U,    \
-                     g, parity, list, nlist, seed, sweep, delta, n_hit, beta_nc, w_t, w_s, partials)
+                     g, parity, list ? 0 : sweep_tw(g), list, nlist, seed, sweep, delta, n_hit, beta_nc, w_t, w_s, partials)
   if (mu == 0) SU2_SWEEP(0);
   else if (mu == 1) SU2_SWEEP(1);
   else if (ND > 2 && mu == 2) SU2_SWEEP((ND > 2 ? 2 : 0));
