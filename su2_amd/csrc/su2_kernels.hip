@@ -973,9 +973,23 @@ template <class G> static bool launch_fused_g(const FusedLaunch &L, hipStream_t 
 }
 
 // SU2GPU_GENFUSE = 0: device momenta always drawn by their own launch
-static int genfuse_pref() {
+int genfuse_pref() {
   static int v = -1;
   if (v < 0) v = env_int("SU2GPU_GENFUSE", 1);
+  return v;
+}
+
+int plq_pref() {
+  static int v = -2;
+  if (v == -2) {
+    int p = env_int("SU2GPU_PLQ", -1);
+    if (p < 0)
+      for (const char *n : {"SU2GPU_TBLOCK", "SU2GPU_NT", "SU2GPU_ZG", "SU2GPU_XWALK", "SU2GPU_TW",
+                            "SU2GPU_TWC", "SU2GPU_TWCZ", "SU2GPU_TWW", "SU2GPU_TWA", "SU2GPU_ZS",
+                            "SU2GPU_FASTSHAPE", "SU2GPU_FUSED"})
+        if (getenv(n)) p = 0;
+    v = p < 0 ? -1 : (p != 0);
+  }
   return v;
 }
 

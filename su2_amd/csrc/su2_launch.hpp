@@ -68,6 +68,11 @@ bool launch_fused(int group, int prec, const FusedLaunch &L, hipStream_t st);
 bool launch_plq(int group, int prec, const FusedLaunch &L, hipStream_t st);
 int plq_partials(int group, int prec, const Geo &geo);
 bool plq_ok(int group, int prec, const Geo &geo, int flags);
+// SU2GPU_PLQ: 0 the shared-plaquette step off, 1 wherever its layout applies, -1 (not
+// set) where it is the faster step; a switch of the staple steps that is set turns it
+// off unless SU2GPU_PLQ is set too.  genfuse_pref: SU2GPU_GENFUSE.
+int plq_pref();
+int genfuse_pref();
 // whether a fused launch of this lattice with these flags runs the specialised
 // step that reads and writes the half-field layout (FP64 SU(2) d = 4,
 // isotropic, specialised launch layout)

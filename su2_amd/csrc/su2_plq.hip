@@ -24,7 +24,8 @@ template <class G> int plq_percu(const PlqGeo &g) {
 // U(1) FP64 12^4 8.9 / 8.1, 16^4 9.1 / 11.1, d = 3 32^3 6.8 / 7.1 us, FP32 16^4 8.1 /
 // 7.7, 20 18 15 27 10.2 / 11.4 us).
 bool plq_geo_for(int group, int prec, const Geo &geo, PlqGeo &g) {
-  if (geo.V < (prec == 0 ? 32768 : 98304)) return false;
+  const int pref = plq_pref();
+  if (pref == 0 || (pref < 0 && geo.V < (prec == 0 ? 32768 : 98304))) return false;
   if (!make_plq_rows(geo.L, geo.nd, geo.V, g)) return false;
   const int percu = group == 1 ? (prec == 0 ? plq_percu<PlqSU2<double>>(g) : plq_percu<PlqSU2<float>>(g))
                                : (prec == 0 ? plq_percu<PlqU1<double>>(g) : plq_percu<PlqU1<float>>(g));
@@ -73,7 +74,7 @@ int plq_partials(int group, int prec, const Geo &geo) {
 
 bool launch_plq(int group, int prec, const FusedLaunch &L, hipStream_t st) {
   if (L.c.flags & (F_ROUND | F_R32L | F_R32P)) return false;
-  if (L.gen && !(L.Uout && (L.c.flags & F_ACCUM))) return false;
+  if (L.gen && !(genfuse_pref() && L.Uout && (L.c.flags & F_ACCUM))) return false;
   if (L.in_half && L.Uout && !L.out_half) return false;  // half -> record steps are not built
   PlqGeo g;
   if (!plq_geo_for(group, prec, L.geo, g)) return false;
