@@ -304,10 +304,15 @@ __global__ __launch_bounds__(PLQ_NT, 2) void k_clover_plq(const quat<T> *__restr
   }
 }
 
+// Not where more than half of the lanes of many blocks hold no site (planes y z of
+// few sites; this / the kernel of the other groups, energy_density in FP64, x y z t):
+// 64 5 5 64 33.9 / 31.9, 64 3 3 64 34.4 / 27.6, 128 1 2 256 95 / 27.6 us; 64 6 6 64 34.0 / 35.8 us;
+// up to 131072 lanes the launches count: 32 5 5 32 24.0 / 27.4, 32 1 2 32 23.6 / 25.3, 32 4 4
+// 64 27.2 / 27.0 us.
 template <typename T> bool clv_geo(const Geo &geo, PlqGeo &g) {
   // FP64: three waves per block, so that two blocks' LDS fits a CU
   const int threads = sizeof(T) == 8 ? 192 : PLQ_NT;
-  if (geo.nd != 4 || !make_plq_rows(geo.L, 4, geo.V, g, threads)) return false;
+  if (geo.nd != 4 || !make_plq_rows(geo.L, 4, geo.V, g, threads) || !plq_full(g)) return false;
   const int waves = (int)plq_threads(g) / 64;
   const int percu = std::max(1, std::min(8 / waves, (int)(160 * 1024 / clv_lds<T>(g))));
   return make_plq_chunks(percu, CUS, g);

@@ -20,8 +20,10 @@
 // two trips inside their branch (carried across the barrier they cost 70 spills).
 // One stage, two-pass form -> this: 24^4 57.2 -> 38.1 us (2.6 TB/s of the 101 MB),
 // 32^4 181.6 -> 109.7, 20x18x15x27 31.2 -> 22.3, 16^4 21.7 -> 14.0, 12^4 19.7 -> 12.0, 8^4 18.1 ->
-// 10.3; no size measured slower, so every lattice the layout takes uses
-// it.  FP64 keeps the two passes: its registers would not fit two waves.
+// 10.3; planes y z of few sites, which leave most lanes idle, keep the two passes where
+// there are many (a stage with its share of the forward pass, this / two passes: 64 5 5 64
+// 58 / 54, 64 2 2 64 38 / 35, 128 1 2 256 113 / 47 us; 64 6 6 64 65 / 67, 32 5 5 32 39 / 45, 32 2 2 32 23 /
+// 27 us).  FP64 keeps the two passes: its registers would not fit two waves.
 #include "su2_flow_adj.hpp"
 #include "su2_md_plq.hpp"
 
@@ -363,7 +365,7 @@ __global__ __launch_bounds__(PLQ_NT) void k_flow_first_adj(const float *__restri
 }
 
 bool flp_geo(const Geo &geo, PlqGeo &g) {
-  if (geo.nd != 4 || !make_plq_rows(geo.L, 4, geo.V, g)) return false;
+  if (geo.nd != 4 || !make_plq_rows(geo.L, 4, geo.V, g) || !plq_full(g)) return false;
   const int waves = (int)plq_threads(g) / 64;
   return make_plq_chunks(std::max(1, std::min(12 / waves, (int)(160 * 1024 / flp_lds(g)))), CUS, g);
 }

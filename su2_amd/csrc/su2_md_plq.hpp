@@ -167,6 +167,17 @@ inline bool make_plq_rows(const int L[4], int nd, int V, PlqGeo &g, int threads 
   return true;
 }
 
+// share of the lanes that hold a site
+inline double plq_fill(const PlqGeo &g) {
+  return (double)g.nrows * g.L[g.nd - 1] / ((double)g.nyb * plq_threads(g));
+}
+
+// lanes mostly in use, or a launch so small that idle ones do not show (measured where
+// it is used)
+inline bool plq_full(const PlqGeo &g) {
+  return plq_fill(g) >= 0.5 || (double)g.nb3 * plq_threads(g) * g.L[0] <= 131072.0;
+}
+
 // The t-chunks where `percu` blocks are resident on each of `cus` CUs.  A slice
 // of a resident round costs a latency and a share per resident wave, in the
 // ratio 2 : 1 (FP32 32^4, measured: chunks of 8 slices, 8 waves per CU, 55.7 us;

@@ -20,13 +20,28 @@ template <class G> int plq_percu(const PlqGeo &g) {
 // (FP64) and 98304 sites (FP32) those are as fast or faster: a launch is bound by
 // its chain of memory round trips, of which this step has two more (FP64 step
 // with events, this / staples: 12^4 10.2 / 9.8, 16^4 12.3 / 13.1, d = 3 32^3 8.5 /
-// 8.7 us; FP32: 16^4 10.5 / 9.7, 20^4 15.8 / 16.2, d = 3 21 59 79 10.1 / 10.3 us;
-// U(1) FP64 12^4 8.9 / 8.1, 16^4 9.1 / 11.1, d = 3 32^3 6.8 / 7.1 us, FP32 16^4 8.1 /
-// 7.7, 20 18 15 27 10.2 / 11.4 us).
+// 8.7 us; FP32: 16^4 10.5 / 9.7, d = 3 48^3 8.8 / 9.1 us; U(1) FP64 12^4 8.9 / 8.1, 16^4
+// 9.1 / 11.1, d = 3 32^3 6.8 / 7.1 us, FP32 16^4 8.1 / 7.7, 20 18 15 27 10.2 / 11.4 us).
+// FP32 SU(2) in d = 4 counts 140000 sites' worth of full lanes (x y z t, steps of a
+// trajectory: 18^4 13.4 / 11.7, 40 10 10 40 16.4 / 14.6, 20^4 14.6 / 14.9, 24^4 24.1 / 24.9,
+// 28^4 41.2 / 45.6 us; 24 24 24 32 33.8 / 30.9 and 32^4 58.4 / 55.5 are its two slower ones).
+//
+// Rows that leave lanes idle (few sites per x plane) cost as much as full ones.  The
+// least share of lanes with a site, this / staples on both sides of the line (x y z t):
+// SU(2) FP64 0.6: 15 5 planes 0.59 11.8 / 11.2, 5 5 0.39 34.9 / 33.6, 3 3 0.14 56.2 / 26.1, 1 2
+// 0.03 89 / 48 us; 9 9 0.63 14.1 / 16.9, 9 5 0.70 9.4 / 11.4 us.  SU(2) FP32 0.7: 9 9 51.9 /
+// 48.6, 6 7 0.66 51.7 / 49.3; 7 7 0.77 52.9 / 58.1, 11 11 0.95 56.3 / 72.3 us.  U(1) FP64 0.35:
+// 4 4 0.25 10.6 / 8.9, 25.7 / 25.5; 5 5 7.8 / 8.7, 27.5 / 37.2 us; FP32 0.5: 5 6 0.47 9.3 / 8.9;
+// 6 6 0.56 9.4 / 9.9, 9 9 13.2 / 18.1 us.
 bool plq_geo_for(int group, int prec, const Geo &geo, PlqGeo &g) {
   const int pref = plq_pref();
-  if (pref == 0 || (pref < 0 && geo.V < (prec == 0 ? 32768 : 98304))) return false;
-  if (!make_plq_rows(geo.L, geo.nd, geo.V, g)) return false;
+  if (pref == 0 || !make_plq_rows(geo.L, geo.nd, geo.V, g)) return false;
+  if (pref < 0) {
+    const double fill = plq_fill(g);
+    if (geo.V < (prec == 0 ? 32768 : 98304)) return false;
+    if (group == 1 && prec == 1 && geo.nd == 4 && geo.V * fill < 140000) return false;
+    if (fill < (group == 1 ? (prec == 0 ? 0.6 : 0.7) : (prec == 0 ? 0.35 : 0.5))) return false;
+  }
   const int percu = group == 1 ? (prec == 0 ? plq_percu<PlqSU2<double>>(g) : plq_percu<PlqSU2<float>>(g))
                                : (prec == 0 ? plq_percu<PlqU1<double>>(g) : plq_percu<PlqU1<float>>(g));
   return make_plq_chunks(percu, CUS, g);

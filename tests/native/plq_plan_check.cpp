@@ -43,6 +43,26 @@ int main() {
                 return 2;
               }
             }
+  // the share of lanes that hold a site, planes y z
+  const struct {
+    int y, z;
+    double fill;
+  } planes[] = {{3, 3, 9.0 / 64}, {4, 4, 16.0 / 64}, {1, 2, 2.0 / 64}, {9, 9, 81.0 / 128},
+                {32, 32, 1.0},    {24, 24, 1.0},     {8, 8, 1.0},      {20, 20, 400.0 / 448},
+                {5, 61, 305.0 / 320}};
+  for (const auto &q : planes) {
+    const int L[4] = {16, 4, q.y, q.z};
+    PlqGeo g;
+    if (!make_plq_rows(L, 4, 64 * q.y * q.z, g)) return 5;
+    if (std::fabs(plq_fill(g) - q.fill) > 1e-12) {
+      printf("%d %d: %f against %f\n", q.y, q.z, plq_fill(g), q.fill);
+      return 6;
+    }
+    // 64 planes: small enough to take either way, 64 t slices of 64 are not
+    if (!plq_full(g)) return 7;
+    const int M[4] = {64, 64, q.y, q.z};
+    if (!make_plq_rows(M, 4, 4096 * q.y * q.z, g) || plq_full(g) != (q.fill >= 0.5)) return 8;
+  }
   const int L[4] = {1 << 20, 4, 8, 1};
   const auto t0 = std::chrono::steady_clock::now();
   long sum = 0;

@@ -57,7 +57,8 @@ def _replay(U, dims, xi):
     return np.stack(out, -2).reshape(-1, 3)
 
 
-@pytest.mark.parametrize("dims,xi", [((24, 16, 18, 16, 4), 1.0), ((16, 16, 32, 17, 4), 1.7),
+# sizes that the dispatch gives to the step
+@pytest.mark.parametrize("dims,xi", [((24, 22, 22, 16, 4), 1.0), ((16, 16, 32, 24, 4), 1.7),
                                      ((64, 32, 1, 64, 3), 1.0)])
 def test_fp32_force_error(oracle, dims, xi):
     U = oracle.hotstart(1, dims, 20251, 0.4).astype(np.float32).astype(np.float64)

@@ -1,7 +1,7 @@
 """The plan of the shared-plaquette step on the host (tests/native/plq_plan_check.cpp): the
 chunk choice equals a plain sum over the rounds and takes microseconds also for a lattice
 long in t (it is made at every launch: 30 us for 2^20 slices; 1 ms is the bound, the plain
-sum takes 6)."""
+sum takes 6), and the share of lanes in use."""
 import os
 import subprocess
 
