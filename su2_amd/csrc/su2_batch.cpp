@@ -70,18 +70,14 @@ struct su2gpu_batch {
       maxpairs = 0;
   // active[3 t + k]: leading link tiles of part k whose lattices still run at tick t
   std::vector<int> active;
-  // the d = 4 part on the shared-plaquette tiles: plans of falling size, tick t
-  // runs the first `count` tiles of plan ptick[t] (-1: its link tiles)
+  // the d = 4 part on the shared-plaquette tiles (BatchPlqTicks): plans of falling size
   struct PlqPlan {
     void *geos = nullptr;
     int2 *tiles = nullptr;
     unsigned threads = 0, lds = 0;
   };
   std::vector<PlqPlan> plans;
-  struct PlqTick {
-    int plan = -1, count = 0;
-  };
-  std::vector<PlqTick> ptick;
+  std::vector<su2k::BatchPlqTicks::Tick> ptick;
   double *partials = nullptr, *dsums = nullptr, *hsums = nullptr;
   uint64_t *dtraj = nullptr, *htraj = nullptr;
   double *staging = nullptr, *hstage = nullptr;
@@ -115,39 +111,24 @@ void free_plans(B *b) {
   b->plans.clear();
 }
 
-// The shared-plaquette tiles of the d = 4 part, from how many running sites on its
-// ticks take them.  The slices of a chunk are chosen for the lattices still
-// running: a new plan whenever their sites fell below three quarters of the last
-// plan's.
+// the shared-plaquette tiles of the d = 4 part (plan_batch_plq) on the device
 int build_plq(B *b, const std::vector<size_t> &order) {
   free_plans(b);
-  b->ptick.assign(b->maxpairs + 1, B::PlqTick{});
   std::vector<size_t> part;
   for (size_t l : order)
     if (b->lat[l].spec == 4) part.push_back(l);
-  double planned = 0.0;
-  std::vector<int> end;
-  for (int t = 0; t <= b->maxpairs; ++t) {
-    while (!part.empty() && b->lat[part.back()].npairs < t) part.pop_back();
-    double run = 0.0;
-    for (size_t l : part) run += b->lat[l].geo.V;
-    if (run < su2k::batch_plq_sites(b->prec)) break;
-    if (b->plans.empty() || run < 0.75 * planned) {
-      su2k::BatchPlqPlan p;
-      if (!su2k::plan_batch_plq(b->prec, b->ncu, b->lat, part, p)) break;
-      b->plans.emplace_back();
-      auto &q = b->plans.back();
-      q.threads = p.threads;
-      q.lds = p.lds;
-      BH(hipMalloc(&q.tiles, p.tiles.size() * sizeof(int2)));
-      BH(hipMemcpy(q.tiles, p.tiles.data(), p.tiles.size() * sizeof(int2), hipMemcpyHostToDevice));
-      BH(hipMalloc(&q.geos, p.geos.size()));
-      BH(hipMemcpy(q.geos, p.geos.data(), p.geos.size(), hipMemcpyHostToDevice));
-      planned = run;
-      end.assign(b->lat.size(), 0);
-      for (size_t i = 0; i < p.tiles.size(); ++i) end[p.tiles[i].x] = (int)i + 1;
-    }
-    b->ptick[t] = {(int)b->plans.size() - 1, end[part.back()]};
+  su2k::BatchPlqTicks ticks;
+  su2k::plan_batch_plq(b->prec, b->ncu, b->lat, part, b->maxpairs, ticks);
+  b->ptick = ticks.tick;
+  for (const auto &p : ticks.plans) {
+    b->plans.emplace_back();
+    auto &q = b->plans.back();
+    q.threads = p.threads;
+    q.lds = p.lds;
+    BH(hipMalloc(&q.tiles, p.tiles.size() * sizeof(int2)));
+    BH(hipMemcpy(q.tiles, p.tiles.data(), p.tiles.size() * sizeof(int2), hipMemcpyHostToDevice));
+    BH(hipMalloc(&q.geos, p.geos.size()));
+    BH(hipMemcpy(q.geos, p.geos.data(), p.geos.size(), hipMemcpyHostToDevice));
   }
   return SU2GPU_OK;
 }
@@ -279,7 +260,7 @@ int enqueue(B *b, bool devmom, Rec *rec = nullptr) {
   fin();
   const int flags = (b->prec == 1) ? (su2k::F_COMPENSATED | su2k::F_RESTORE) : 0;
   auto tick = [&](int t, int part, hipStream_t st) {
-    const auto pt = part == 0 ? b->ptick[t] : B::PlqTick{};
+    const auto pt = part == 0 ? b->ptick[t] : su2k::BatchPlqTicks::Tick{};
     if (pt.plan >= 0) {
       const auto &q = b->plans[pt.plan];
       su2k::launch_batch_plq(b->prec, b->dlat, q.geos, q.tiles, pt.count, b->nltiles, b->ar, t,
@@ -287,7 +268,7 @@ int enqueue(B *b, bool devmom, Rec *rec = nullptr) {
     } else {
       su2k::launch_batch_tick(b->prec, b->dlat, b->dltiles, b->nltiles, b->nspec4, b->nspec3,
                               b->ar, t, flags, b->partials, b->grid, b->block, st, part,
-                              &b->active[3 * t]);
+                              b->active[3 * t + part]);
     }
   };
   if (!rec && b->concurrent) {

@@ -285,27 +285,25 @@ __global__ __launch_bounds__(256) void k_batch_reduce(const BLat *__restrict__ l
 // ------------------------------------------------------------- launchers ----
 void launch_batch_tick(int prec, const BLat *lats, const int2 *tiles, int ntiles, int n4, int n3,
                        const BArenas &ar, int tick, int flags, double *partials, int grid,
-                       int block, hipStream_t st, int only, const int *active) {
-  const int parts[3][2] = {{0, n4}, {n4, n3}, {n4 + n3, ntiles - n4 - n3}};
-  for (int k = 0; k < 3; ++k) {
-    const int t0 = parts[k][0];
-    const int n = active ? (active[k] < parts[k][1] ? active[k] : parts[k][1]) : parts[k][1];
-    if (n <= 0 || (only >= 0 && k != only)) continue;
-    const dim3 g(grid < n ? grid : n), bl(block);
+                       int block, hipStream_t st, int part, int active) {
+  const int t0 = part == 0 ? 0 : part == 1 ? n4 : n4 + n3;
+  const int all = part == 0 ? n4 : part == 1 ? n3 : ntiles - n4 - n3;
+  const int n = active < all ? active : all;
+  if (n <= 0) return;
+  const dim3 g(grid < n ? grid : n), bl(block);
 #define SU2_TICK(T, S) \
   hipLaunchKernelGGL((k_batch_tick<T, S>), g, bl, 0, st, lats, tiles, t0, n, ntiles, ar, tick, flags, partials)
 #define SU2_TICK3(T)            \
-  if (k == 0) SU2_TICK(T, 4);   \
-  else if (k == 1) SU2_TICK(T, 3); \
+  if (part == 0) SU2_TICK(T, 4);   \
+  else if (part == 1) SU2_TICK(T, 3); \
   else SU2_TICK(T, 0)
-    if (prec == 0) {
-      SU2_TICK3(double);
-    } else {
-      SU2_TICK3(float);
-    }
+  if (prec == 0) {
+    SU2_TICK3(double);
+  } else {
+    SU2_TICK3(float);
+  }
 #undef SU2_TICK3
 #undef SU2_TICK
-  }
 }
 void launch_batch_plaq(int prec, const BLat *lats, const int2 *tiles, int ntiles, const BArenas &ar,
                        int use_final, int row, int rowlen, double *partials, int grid, int block,

@@ -68,28 +68,36 @@ __device__ inline void batch_tick_coef(const BLat &L, int tick, int flags, Fused
 
 // ltiles: (lattice, site_start * 4 + mu): those of the specialised SU(2)
 // lattices in d = 4 ([0, n4)), then in d = 3 ([n4, n4 + n3)), then the rest;
-// partial rows are nltiles long.  One launch per part (at most `grid` blocks
-// each), so that each part has its own register budget; only >= 0 launches
-// that part alone (0: d = 4, 1: d = 3, 2: the rest).  active (optional): the
-// number of leading tiles of each part that belong to lattices still running
-// at this tick (each part's lattices are ordered by step count, longest
-// first); the launch covers only those.
+// partial rows are nltiles long.  One launch of at most `grid` blocks for one part
+// (0: d = 4, 1: d = 3, 2: the rest), so that each part has its own register budget.
+// active: the number of the part's leading tiles that belong to lattices still running
+// at this tick (each part's lattices are ordered by step count, longest first).
 void launch_batch_tick(int prec, const BLat *lats, const int2 *ltiles, int nltiles, int n4, int n3,
                        const BArenas &ar, int tick, int flags, double *partials, int grid,
-                       int block, hipStream_t st, int only = -1, const int *active = nullptr);
-// A tick of the specialised d = 4 part with the shared-plaquette step
-// (su2_batch_plq.hip): its tiles (lattice, block of the lattice's layout) and the
-// layouts (PlqGeo, one per lattice of the batch), for the lattices `part` in that
-// order.  False where the link tiles are kept.
+                       int block, hipStream_t st, int part, int active);
+// The ticks of the specialised d = 4 part with the shared-plaquette step
+// (su2_batch_plq.hip).  A plan: tiles (lattice, block of the lattice's layout) in the
+// lattices' order and the layouts (PlqGeo, one per lattice of the batch).
 struct BatchPlqPlan {
   unsigned threads = 0, lds = 0;
   std::vector<char> geos;
   std::vector<int2> tiles;
 };
-bool plan_batch_plq(int prec, int ncu, const std::vector<BLat> &lat, const std::vector<size_t> &part,
-                    BatchPlqPlan &p);
-// running sites from which a tick takes it: the single lattice's line
-constexpr int batch_plq_sites(int prec) { return prec == 0 ? 32768 : 98304; }
+// tick t runs the first `count` tiles of plan `plan` (-1: its link tiles).  The slices
+// of a chunk are chosen for the lattices still running: a new plan whenever their sites
+// fell below three quarters of the last plan's.
+struct BatchPlqTicks {
+  struct Tick {
+    int plan = -1, count = 0;
+  };
+  std::vector<BatchPlqPlan> plans;
+  std::vector<Tick> tick;
+};
+// `part`: the part's lattices, those with more steps first.  A tick whose running
+// lattices are too few, do not all fit the layout or leave too many lanes idle keeps
+// the link tiles.
+void plan_batch_plq(int prec, int ncu, const std::vector<BLat> &lat, const std::vector<size_t> &part,
+                    int maxpairs, BatchPlqTicks &out);
 void launch_batch_plq(int prec, const BLat *lats, const void *geos, const int2 *tiles, int count,
                       int rowlen, const BArenas &ar, int tick, int flags, double *partials,
                       unsigned threads, unsigned lds, hipStream_t st);

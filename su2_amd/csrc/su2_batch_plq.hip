@@ -58,32 +58,28 @@ __global__ __launch_bounds__(PLQ_NT, plq_occ<G>()) void k_batch_plq(
   }
 }
 
+// the layouts and chunks of the first n lattices of `part`
 template <class G>
 static bool plan_part(int ncu, const std::vector<BLat> &lat, const std::vector<size_t> &part,
-                      BatchPlqPlan &p) {
+                      size_t n, BatchPlqPlan &p) {
   std::vector<PlqGeo> geo(lat.size());
   p = BatchPlqPlan{};
-  double sites = 0.0, lanes = 0.0;
+  const std::vector<size_t> run(part.begin(), part.begin() + n);
   int maxT = 1;
-  for (size_t l : part) {
+  for (size_t l : run) {
     PlqGeo &g = geo[l];
     if (!make_plq_rows(lat[l].geo.L, 4, lat[l].geo.V, g)) return false;
     p.threads = std::max(p.threads, plq_threads(g));
     p.lds = std::max(p.lds, (unsigned)plq_lds<G, 4>(g));
-    sites += g.V;
-    lanes += (double)g.nb3 * plq_threads(g) * g.L[0];
     maxT = std::max(maxT, g.L[0]);
   }
-  // the step gains up to a factor 1.5 on full waves: not where the rows fill
-  // less than two thirds of them
-  if (part.empty() || lanes > 1.5 * sites) return false;
   // slices per chunk for all lattices together: the cost of make_plq_chunks
   const int percu = std::max(1, std::min(plq_occ<G>() * 4 * 64 / (int)p.threads, (int)(160 * 1024 / p.lds)));
   double cost = 1e300;
   int best = 1;
   for (int Tc = 1; Tc <= maxT; ++Tc) {
     double nb = 0.0, waves = 0.0, c = 0.0;
-    for (size_t l : part) {
+    for (size_t l : run) {
       const PlqGeo &g = geo[l];
       const double n = (double)g.nb3 * ((g.L[0] + Tc - 1) / Tc);
       nb += n;
@@ -97,9 +93,12 @@ static bool plan_part(int ncu, const std::vector<BLat> &lat, const std::vector<s
       best = Tc;
     }
   }
-  for (size_t l : part) {
+  for (size_t l : run) {
     PlqGeo &g = geo[l];
     g.Tc = std::min(best, g.L[0]);
+    // longer chunks where a small lattice would have more blocks than entries for
+    // their sums
+    while (g.Tc < g.L[0] && g.nb3 * ((g.L[0] + g.Tc - 1) / g.Tc) > lat[l].nltiles) ++g.Tc;
     g.nchunk = (g.L[0] + g.Tc - 1) / g.Tc;
     if ((uint64_t)g.nb3 * g.nchunk * g.nb3 >= (1ull << 32)) return false;
     g.mnyb = fast_div_magic((uint32_t)g.nyb);
@@ -112,10 +111,46 @@ static bool plan_part(int ncu, const std::vector<BLat> &lat, const std::vector<s
   return true;
 }
 
-bool plan_batch_plq(int prec, int ncu, const std::vector<BLat> &lat, const std::vector<size_t> &part,
-                    BatchPlqPlan &p) {
-  return prec == 0 ? plan_part<PlqSU2<double>>(ncu, lat, part, p)
-                   : plan_part<PlqSU2<float>>(ncu, lat, part, p);
+// running sites from which a tick takes these tiles
+static double min_sites(int prec) { return prec == 0 ? 32768 : 98304; }
+// lanes that may go with a site: the step gains up to a factor 1.5 on full waves
+static double max_lanes(int) { return 1.5; }
+
+void plan_batch_plq(int prec, int ncu, const std::vector<BLat> &lat, const std::vector<size_t> &part,
+                    int maxpairs, BatchPlqTicks &out) {
+  out.plans.clear();
+  out.tick.assign(maxpairs + 1, BatchPlqTicks::Tick{});
+  // of the first n lattices: sites, lanes, and those the layout does not take
+  std::vector<double> sites(1, 0.0), lanes(1, 0.0);
+  std::vector<int> bad(1, 0);
+  for (size_t l : part) {
+    PlqGeo g;
+    const bool ok = make_plq_rows(lat[l].geo.L, 4, lat[l].geo.V, g) && g.nb3 <= lat[l].nltiles;
+    sites.push_back(sites.back() + lat[l].geo.V);
+    lanes.push_back(lanes.back() + (ok ? (double)g.nb3 * plq_threads(g) * g.L[0] : 0.0));
+    bad.push_back(bad.back() + (ok ? 0 : 1));
+  }
+  size_t n = part.size();
+  double tried = 0.0;  // sites at the last attempt at a plan, and whether there is one for them
+  bool have = false;
+  std::vector<int> end;
+  for (int t = 0; t <= maxpairs; ++t) {
+    while (n > 0 && lat[part[n - 1]].npairs < t) --n;
+    if (n == 0 || sites[n] < min_sites(prec)) break;
+    if (bad[n] > 0 || lanes[n] > max_lanes(prec) * sites[n]) continue;
+    if (tried == 0.0 || sites[n] < 0.75 * tried) {
+      tried = sites[n];
+      BatchPlqPlan p;
+      have = prec == 0 ? plan_part<PlqSU2<double>>(ncu, lat, part, n, p)
+                       : plan_part<PlqSU2<float>>(ncu, lat, part, n, p);
+      if (have) {
+        end.assign(lat.size(), 0);
+        for (size_t i = 0; i < p.tiles.size(); ++i) end[p.tiles[i].x] = (int)i + 1;
+        out.plans.push_back(std::move(p));
+      }
+    }
+    if (have) out.tick[t] = {(int)out.plans.size() - 1, end[part[n - 1]]};
+  }
 }
 
 void launch_batch_plq(int prec, const BLat *lats, const void *geos, const int2 *tiles, int count,
