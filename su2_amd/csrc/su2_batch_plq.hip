@@ -111,10 +111,14 @@ static bool plan_part(int ncu, const std::vector<BLat> &lat, const std::vector<s
   return true;
 }
 
-// running sites from which a tick takes these tiles
+// Running sites from which a tick takes these tiles, and the lanes that may go with a
+// site.  Batches of equal members on one GPU, a trajectory of 20 steps (these tiles /
+// link tiles): FP64 full waves 32 x 8^4 423 / 571 us, 4 x 16^4 697 / 962, three quarters full
+// 16 x 12^4 917 / 1214, 24 x 7^4 336 / 336; FP32 full waves 32 x 8^4 292 / 307, 8 x 16^4 748 / 831,
+// three quarters full 8 x 12^4 410 / 359, 32 x 12^4 1118 / 1076, 64 x 7^4 410 / 381, 16 x 10^4 392 /
+// 355 us.  The mixed ensemble of 8^4, 12^4 and 16^4 has 1.08 lanes to a site.
 static double min_sites(int prec) { return prec == 0 ? 32768 : 98304; }
-// lanes that may go with a site: the step gains up to a factor 1.5 on full waves
-static double max_lanes(int) { return 1.5; }
+static double max_lanes(int prec) { return prec == 0 ? 1.5 : 1.2; }
 
 void plan_batch_plq(int prec, int ncu, const std::vector<BLat> &lat, const std::vector<size_t> &part,
                     int maxpairs, BatchPlqTicks &out) {

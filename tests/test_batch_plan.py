@@ -57,3 +57,10 @@ def test_member_outside_the_layout_counts_only_while_it_runs(plan):
     # planes that leave three quarters of the lanes idle likewise
     ticks = plan(0, rest + [((16, 4, 4, 256), 12)])
     assert [p >= 0 for p, _, _ in ticks] == [False] * 13 + [True] * 18
+
+
+def test_lanes_to_a_site(plan):
+    # three quarters of the lanes: FP64 takes them, FP32 does not
+    assert plan(0, [((12, 12, 12, 12), 5)] * 8)[0][0] == 0
+    assert plan(1, [((12, 12, 12, 12), 5)] * 8)[0][0] == -1
+    assert plan(1, [((8, 8, 8, 8), 5)] * 32)[0][0] == 0
