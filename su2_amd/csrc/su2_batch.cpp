@@ -381,10 +381,14 @@ int ensure_stage(B *b, size_t n) {
   return SU2GPU_OK;
 }
 
-// a download of up to DIRECT_BYTES into pinned memory goes there straight from the kernel that converts it, without
-// a staging copy (the 224 members of the mixed ensemble, 173 MB in all: 8.2 -> 6.0
-// ms, 3.3 at the link's rate); larger ones, and pageable memory, are staged
-constexpr size_t DIRECT_BYTES = 4 << 20;
+// a download of up to DIRECT_BYTES into pinned memory goes there straight from the
+// kernel that converts it, without a staging copy (the 224 members of the mixed
+// ensemble, 173 MB in all: 8.2 -> 6.0 ms, 3.3 at the link's rate); larger ones, and
+// pageable memory, are staged.  The copy engine's rate is some per cent higher: this /
+// staged, SU(2) 8^4 (0.5 MB) 21 / 30 us, 16^4 (8.4 MB) 163 / 177, 20^4 (20 MB) 387 / 391, 24^4 (42 MB)
+// 790 / 781, 32^4 (134 MB) 2470 / 2404; U(1) d = 2 64^2 13 / 22, 512^2 (4.2 MB) 87 / 96, 1024^2 (17 MB)
+// 320 / 326; both forms alike.
+constexpr size_t DIRECT_BYTES = 20 << 20;
 
 std::string signature(const B *b) {
   std::ostringstream ss;
