@@ -24,17 +24,18 @@ int main() {
     top(ec[x > 1.0], c - cosl(a));
     top(es[x > 1.0], s - sinl(a) / a);
   }
-  // angles up to 3e4, and the tiny ones' relative error
-  for (int i = -400000; i <= 400000; ++i) {
-    const double a = i * 0.0750000001;
-    int j;
-    const double r = plq_reduce(a, j);
-    double c, s;
-    plq_sincos(r, c, s);
-    plq_quadrant(j, c, s);
-    top(rc, c - cosl((long double)a));
-    top(rs, s - sinl((long double)a));
-  }
+  // angles up to 3e4, to 1e8 and to 4e14
+  for (double f : {1.0, 3333.33, 1.3e10})
+    for (int i = -400000; i <= 400000; ++i) {
+      const double a = i * 0.0750000001 * f;
+      int j;
+      const double r = plq_reduce(a, j);
+      double c, s;
+      plq_sincos(r, c, s);
+      plq_quadrant(j, c, s);
+      top(rc, c - cosl((long double)a));
+      top(rs, s - sinl((long double)a));
+    }
   printf("%.4Lf %.4Lf %.4Lf %.4Lf %.4Lf %.4Lf\n", ec[0] / u, es[0] / u, ec[1] / u, es[1] / u, rc / u,
          rs / u);
   return 0;

@@ -6,8 +6,9 @@ Derived bounds.  cos_sinc_fp64 up to x = 1: the last fused step rounds once, 1/2
 of 1 1/2 units, 3/4 unit at x = 1, and the terms left out are below 0.1: 1.35, taken as
 1.5 (a cosine series one power shorter leaves out 1.5 units alone).  Up to x = 12 the
 root's half ulp is 2 units: 3.5 and, divided by a, 2.5.  Reduced sine and cosine of
-angles up to 3e4: the reduced angle's rounding is half an ulp, the second part of pi/2
-is rounded at 2^-87 and multiplied by up to 2^15: 1 1/2."""
+angles up to 4e14: the reduced angle's rounding is half an ulp, the second part of pi/2
+is rounded at 2^-87 and multiplied by up to 2^17, that of 2 pi at 2^-105 and by up to 2^46:
+1 1/2."""
 import os
 import subprocess
 
