@@ -1265,7 +1265,7 @@ int observables(L *h, int want, Observables *o) {
   constexpr int R0 = 20;
   su2k::RowList rl;
   int nb = 0;
-  if (want & OBS_E) {
+  if ((want & OBS_E) && su2k::clover_partials(h->group, h->prec, h->geo) > 0) {
     Prof pr(h, "energy_density");
     nb = su2k::launch_clover(h->group, h->prec, h->U[h->cur], h->geo, row(h, R0), h->row_stride,
                              h->stream);
