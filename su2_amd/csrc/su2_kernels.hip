@@ -472,7 +472,9 @@ static int xwalk_pref() {
 // specialised step; default: where the two link fields and the momenta exceed
 // the 256 MB Infinity Cache (48^4 FP32 466 against 496 us, 64^4 1331 against
 // 1446 us; at 32^4, which fits, 79 against 67 us).  2: also non-temporal
-// momentum loads in the FP64 half-field step (default beyond 1 GiB)
+// momentum loads in the FP64 half-field step (default beyond 1 GiB).  Times of the staple
+// steps among themselves, here and at the switches below (launch_fused says which
+// lattices reach them)
 static int nt_pref() {
   static int v = -2;
   if (v == -2) v = env_int("SU2GPU_NT", -1);
@@ -1086,6 +1088,14 @@ static bool launch_first_step_gen(int group, int prec, const FusedLaunch &L, hip
   return true;
 }
 
+// The shared-plaquette step first.  What it leaves to the staple steps (plq_geo_for):
+// d = 2; fewer than 32768 sites (FP64), 98304 (FP32; SU(2) d = 4 140000 of full lanes);
+// planes of the two fastest directions that fill too few lanes, such as 4 x 4; rows of 1
+// and of more than 128 sites; 2^27 sites and more; and every lattice when a switch of
+// the staple steps is set.  So the t-walks, their forms in two chunks, with
+// non-temporal accesses and with the lane exchanges run by themselves for small
+// lattices long in t (8 8 8 32), planes of few sites (64 4 4 64) and 128^4 and beyond; the
+// figures at 32^4, 48^4 and 64^4 beside them compare these steps among themselves.
 bool launch_fused(int group, int prec, const FusedLaunch &L, hipStream_t st) {
   if (fast_level() >= (prec == 0 ? 2 : 1) && launch_plq(group, prec, L, st)) return true;
   if (L.gen) {
