@@ -1,6 +1,6 @@
 // The sine / cosine series of su2_md_plq.hpp against 80-bit arithmetic on the host:
 // largest errors of cos a and sin(a)/a as functions of x = a^2 (cos_sinc_fp64) for x
-// up to 1 and up to 12, and of the reduced sine and cosine, in units of 2^-53.
+// up to 1 and up to 12, and of the reduced sine and cosine of angles up to 3e4 and beyond, in units of 2^-53.
 #include <cmath>
 #include <cstdio>
 
@@ -10,7 +10,7 @@ using namespace su2k;
 
 int main() {
   const long double u = 0x1p-53L;
-  long double ec[2] = {}, es[2] = {}, rc = 0, rs = 0;
+  long double ec[2] = {}, es[2] = {}, rc[2] = {}, rs[2] = {};
   auto top = [](long double &m, long double e) {
     e = fabsl(e);
     if (!(e <= m)) m = e;
@@ -33,10 +33,10 @@ int main() {
       double c, s;
       plq_sincos(r, c, s);
       plq_quadrant(j, c, s);
-      top(rc, c - cosl((long double)a));
-      top(rs, s - sinl((long double)a));
+      top(rc[f > 1.0], c - cosl((long double)a));
+      top(rs[f > 1.0], s - sinl((long double)a));
     }
-  printf("%.4Lf %.4Lf %.4Lf %.4Lf %.4Lf %.4Lf\n", ec[0] / u, es[0] / u, ec[1] / u, es[1] / u, rc / u,
-         rs / u);
+  printf("%.4Lf %.4Lf %.4Lf %.4Lf %.4Lf %.4Lf %.4Lf %.4Lf\n", ec[0] / u, es[0] / u, ec[1] / u,
+         es[1] / u, rc[0] / u, rs[0] / u, rc[1] / u, rs[1] / u);
   return 0;
 }
