@@ -441,8 +441,8 @@ def progress(msg):
 
 def kernel_name(prec, L):
     """Instantiation of the step that a P-then-U launch of the L^4 SU(2) lattice
-    takes, as rocprofv3 names it.  From 32768 (FP64) or 98304 sites (FP32) and up
-    to rows of 128: k_md_plq<group, nd, write U, sums, draw, NT, link in, link out>
+    takes, as rocprofv3 names it.  From 32768 (FP64) or, in full lanes, 140000 sites
+    (FP32, which 20^4 reaches) and up to rows of 128: k_md_plq<group, nd, write U, sums, draw, NT, link in, link out>
     (su2_plq.hip), non-temporal (NT = 2) where the two link fields and the momenta
     exceed 256 MiB; FP64 on the half-field layout where the 3-volume is a
     multiple of 256.  Below: k_md_su2_4d<T, WRITE_U, ACCUM, SPEC, ZS, AN, NT, in,
@@ -454,7 +454,7 @@ def kernel_name(prec, L):
     half = prec == 0 and L ** 3 % 256 == 0
     link = ("su2k::QHalf, su2k::QHalfW" if half
             else f"su2dev::quat<{t}> const*, su2dev::quat<{t}>*")
-    if L ** 4 >= (32768 if prec == 0 else 98304) and L <= 128:
+    if L ** 4 >= (32768 if prec == 0 else 140000) and L <= 128:
         return f"k_md_plq<su2k::PlqSU2<{t}>, 4, true, false, false, {nt}, {link}>"
     if L ** 3 % 256 == 0:
         zs = 1 if 64 % L == 0 else 0

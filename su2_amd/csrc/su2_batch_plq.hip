@@ -8,8 +8,9 @@
 //
 // Bound as the single lattice's step: latency and issue.  The 32 lattices of 8^4,
 // 12^4 and 16^4 of the mixed ensemble (1.05 M sites, FP32, beside the d = 3 and U(1)
-// ticks): 94 -> 69 us at the first tick, 64 with all of them running and 63.3 -> 57
-// on the average of a trajectory.  The same step for the d = 3 part (273000 sites)
+// ticks): 63.3 -> 59.6 us on the average of a trajectory, the first tick, whose sums cost 24
+// spilled registers in FP32, 94 -> 92 us (with 2 waves per SIMD and no spills a trajectory
+// takes as long).  The same step for the d = 3 part (273000 sites)
 // took 25 us where the link tiles take 20: not built.
 #include "su2_batch.hpp"
 #include "su2_md_plq.hpp"

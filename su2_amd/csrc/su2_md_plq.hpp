@@ -33,10 +33,11 @@
 // (links; momenta and edge-row links, which are loaded together while the last
 // planes are evaluated).  FP64: 32^4 143 -> 107 us (565 MB beyond the L2, 5.3
 // TB/s), 48^4 784 -> 518 us (112 B per link at 4.6 TB/s), 40^4 386 -> 287 us,
-// 24^4 48.6 -> 38.9 us, momentum-only 32^4 115 -> 82 us.  FP32: 48^4 384 -> 285
-// us, 40^4 190 -> 151 us, 32^4 58.7 -> 55.7 us (VALU 60 % busy).  U(1), where the
+// 24^4 48.6 -> 38.9 us, momentum-only 32^4 115 -> 82 us.  FP32: 48^4 384 -> 277
+// us, 40^4 188 -> 150 us, 28^4 45.5 -> 41.0 us, 32^4 a tie (55.5 to 61.6 / 58.2 to 61.4
+// us over four cards).  U(1), where the
 // staple form takes seven sine / cosine pairs per link and this one six sines per
-// site and three for x-1: FP64 24^4 33.8 -> 17.8 us, 32^4 85.5 -> 35.2 us, d = 3
+// site and three for x-1: FP64 24^4 33.8 -> 17.8 us (15.2 in a trace, without the events), 32^4 85.5 -> 35.2 us, d = 3
 // 64^3 17.8 -> 10.9 us; FP32 32^4 46.7 -> 24.3 us.  Loading the
 // next slice's first links during the update spills (FP64) and makes the next
 // slice wait for the update's stores, which share the counter of the loads:
@@ -180,8 +181,8 @@ inline bool plq_full(const PlqGeo &g) {
 
 // The t-chunks where `percu` blocks are resident on each of `cus` CUs.  A slice
 // of a resident round costs a latency and a share per resident wave, in the
-// ratio 2 : 1 (FP32 32^4, measured: chunks of 8 slices, 8 waves per CU, 55.7 us;
-// of 6, 12 waves, 59.6; of 4, two rounds, 61.9; FP64 24^4: 4 slices 39, 3 slices
+// ratio 2 : 1 (FP32 32^4, measured: chunks of 8 slices, 8 waves per CU, 58.5 us;
+// of 6, 12 waves, 60.8; of 4, two rounds, 60.3; FP64 24^4: 4 slices 39, 3 slices
 // 43.7, 2 slices 43.2 us), a chunk's first slice a third more (the terms of
 // the slice below it).
 inline bool make_plq_chunks(int percu, int cus, PlqGeo &g) {

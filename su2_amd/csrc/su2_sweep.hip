@@ -95,7 +95,7 @@ __device__ __forceinline__ bool below_exp(double v, double dS) {
 // FP64 SU(2), records of 32 bytes: the loads of one plane at a time (all of a side's
 // take 128 registers and 20 spills: 619 us) and at most 4 blocks on a CU, held
 // by SWEEP_PAD bytes of LDS: with the 7 that the registers allow the blocks' lines
-// push each other out of the L2, 550 against 526 us (5 and 3 blocks: 535, 553).  The cap
+// push each other out of the L2, 550 against 526 us on one card (5 and 3 blocks: 535, 553).  The cap
 // was not slower at any size tried (with / without): 16^4 one hit 65.9 / 67.6, 48^4 one hit
 // 2176 / 2205, ten 2286 / 2474, d = 3 96^3 188 / 198 and 300 / 304, 128^3 532 / 551, d = 2 2048^2
 // 282 / 286, three colours 33^4 741 / 750 us.
