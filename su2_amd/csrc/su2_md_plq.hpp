@@ -37,8 +37,8 @@
 // us, 40^4 188 -> 150 us, 28^4 45.5 -> 41.0 us, 32^4 a tie (55.5 to 61.6 / 58.2 to 61.4
 // us over four cards).  U(1), where the
 // staple form takes seven sine / cosine pairs per link and this one six sines per
-// site and three for x-1: FP64 24^4 33.8 -> 17.8 us (15.2 in a trace, without the events), 32^4 85.5 -> 35.2 us, d = 3
-// 64^3 17.8 -> 10.9 us; FP32 32^4 46.7 -> 24.3 us.  Loading the
+// site and three for x-1: FP64 24^4 33.8 -> 18.9 us (16.4 in a trace, without the events), 32^4 85.5 -> 38.0 us, d = 3
+// 64^3 17.8 -> 11.0 us; FP32 32^4 46.7 -> 24.6 us.  Loading the
 // next slice's first links during the update spills (FP64) and makes the next
 // slice wait for the update's stores, which share the counter of the loads:
 // 137 us at 32^4.
@@ -346,7 +346,7 @@ __host__ __device__ __forceinline__ void plq_sincos(double r, double &c, double 
 __host__ __device__ __forceinline__ double plq_reduce(double a, int &j) {
   if (fabs(a) > 1e5) {
     // whole turns off first, 2 pi in two parts (the sum rounds at 2^-52, an angle of
-    // this size at 2^-37; carrying the second part to the end cost U(1) 24^4 15.2 -> 15.7 us);
+    // this size at 2^-37; carrying the second part to the end for every angle cost U(1) 24^4 0.5 us);
     // beyond 1e15 an angle's own spacing is an eighth and more
     if (fabs(a) > 1e15) a = fmod(a, 6.283185307179586477);
     const double n = rint(a * 0.15915494309189533577);
